@@ -27,10 +27,11 @@ pcx_status fail_with(pcx_status st, const std::string& msg) {
   return st;
 }
 
+// An attribute, not hipGetDeviceProperties: every run asks, and the latter
+// fills a structure of hundreds of fields.
 int device_cus(int device) {
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
-    return prop.multiProcessorCount;
+  int v = 0;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && v > 0) return v;
   return 256;
 }
 
@@ -121,13 +122,69 @@ pcx_status ensure_adjacency(pcx_engine* e) {
   PCX_HIP(hipMalloc(&e->d_adj, adj.size() * sizeof(int32_t)));
   PCX_HIP(hipMemcpy(e->d_adj_off, off.data(), (V + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
   PCX_HIP(hipMemcpy(e->d_adj, adj.data(), adj.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  e->adj_vars = V;
+  e->adj_n = off[V];
   e->adj_version = e->version;
+  return PCX_OK;
+}
+
+// One store through the LDS kernel: up to 48 K propagators, where one workgroup
+// still beats sweeps by the whole device (ms per fixpoint at 1,000 / 16,000 /
+// 48,000 / 74,000 propagators: 0.23 / 0.66 / 1.4 / 1.9 here, 0.95 / 1.9 / 2.0 /
+// 1.6 in sweeps).  Intervals, automatic settings and runs to the fixpoint only.
+constexpr int64_t kLocalSingleProps = 48 * 1024;
+bool single_local(const pcx_engine* e, int64_t nvars) {
+  const pcx_config& c = e->cfg;
+  const int64_t n = (int64_t)e->op.size();
+  return c.domain == PCX_DOMAIN_INTERVAL && c.lds_mode != 0 && c.max_sweeps <= 0 && c.event_driven < 0 &&
+         c.props_per_wave == 0 && c.mark_queue < 0 && n <= kLocalSingleProps && local_fits(c.device, nvars, n);
+}
+
+// The LDS kernel on one store of separate bounds, in memory the device can
+// address; flags may be pinned host memory.  The table and its adjacency
+// records are on the device.
+hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, InstFlags* flags) {
+  LocalJob job{};
+  job.lb = lb;
+  job.ub = ub;
+  job.nvars = nvars;
+  job.n_inst = 1;
+  job.flags = flags;
+  job.adj_off = e->d_adj_off;
+  job.adj_vars = (int32_t)e->adj_vars;
+  job.adj = e->d_adj_rec;
+  return launch_local(Table{e->d_xo, e->d_y, e->d_z, (int64_t)e->op.size()}, job, dom_of(e), e->cfg.device,
+                      device_cus(e->cfg.device), e->stream);
+}
+
+// Its flags as a result: one sweep of the whole table (unless the store was
+// empty to begin with), then the evaluations of the marked rounds.
+pcx_result single_result(const pcx_engine* e, const InstFlags& f) {
+  const int32_t last = std::max(f.changed[0], f.changed[1]);
+  pcx_result r{};
+  r.failed = f.failed_at != kNoFail;
+  r.has_changed = last >= 0;
+  r.sweeps = r.failed ? (int64_t)f.failed_at + 1 : (int64_t)last + 2;
+  r.evals = f.failed_at == -1 ? 0 : (int64_t)e->op.size() + f.marked_evals;
+  return r;
+}
+
+// 16 B per adjacency entry, written by the device from the table it holds.
+pcx_status ensure_adj_records(pcx_engine* e) {
+  pcx_status st = ensure_adjacency(e);
+  if (st != PCX_OK || (e->d_adj_rec && e->adj_rec_version == e->version)) return st;
+  dfree(e->d_adj_rec);
+  PCX_HIP(hipMalloc(&e->d_adj_rec, std::max<int64_t>(e->adj_n, 1) * sizeof(int4)));
+  PCX_HIP(launch_adj_records(Table{e->d_xo, e->d_y, e->d_z, (int64_t)e->op.size()}, e->d_adj, e->adj_n,
+                             e->d_adj_rec, e->stream));
+  e->adj_rec_version = e->version;
   return PCX_OK;
 }
 
 }  // namespace pcx_internal
 
 using pcx_internal::dom_of;
+using pcx_internal::ensure_adj_records;
 using pcx_internal::ensure_adjacency;
 using pcx_internal::sync_table;
 
@@ -146,9 +203,7 @@ int ppw_of(const pcx_engine* e, int64_t m = -1) {
   // plain sweeps unroll at most 512 per wave (batched items go to 2048)
   if (e->cfg.props_per_wave) return m < 0 ? e->cfg.props_per_wave : std::min(e->cfg.props_per_wave, 512);
   if (m < 0) return 512;
-  int cus = 256;
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, e->cfg.device) == hipSuccess) cus = prop.multiProcessorCount;
+  const int cus = pcx_internal::device_cus(e->cfg.device);
   for (int ppw = 512; ppw > 64; ppw /= 2)
     if (m / ((int64_t)kBlock * (ppw / kWave)) >= 2LL * cus) return ppw;
   return 64;
@@ -426,7 +481,80 @@ Subsets run_subsets(const pcx_batch* b) {
   return Subsets{b->d_off, b->compact ? nullptr : b->d_idx};
 }
 
-pcx_status prepare_run(pcx_batch* b, int32_t mode) {
+// A run that starts from the loaded stores, whose load listed the values that
+// differ from the base store (the values instances 0-2 agree on), needs in
+// its first sweep only (a) the member propagators adjacent to a listed value
+// of their instance and (b) the propagators the base store does not satisfy,
+// in every instance that holds them: any other propagator reads in instance
+// k the values it reads in the base store, where it tightens nothing.  These are seeded as the first
+// sweep's marks, which makes that sweep a marked sweep, when their count is
+// under 1/16 of the pairs a full sweep evaluates (and the list is complete).
+// This decides (after the stores' state was taken over into the run); the run
+// launches the seeding (n_unsat propagators listed in d_unsat) with its own
+// event set.
+struct SeedPlan {
+  bool seeded = false;
+  int64_t n_diff = 0, n_unsat = 0;
+};
+pcx_status plan_seed(pcx_batch* b, SeedPlan* plan) {
+  *plan = SeedPlan{};
+  pcx_engine* e = b->e;
+  if (!events_possible(b, PCX_MODE_BATCHED) || b->seeded || !b->run_from_image || !b->diffs_listed ||
+      e->cfg.base_seed == 0)
+    return PCX_OK;
+  // The probe and the counts depend on the image and the table only: runs
+  // from the same image (after resets) reuse them.
+  if (!b->probe_valid || b->probe_version != e->version) {
+    if (!b->d_unsat) PCX_HIP(hipMalloc(&b->d_unsat, b->table_n * sizeof(int32_t)));
+    int32_t* unsat_n = b->d_seedctl + kDiffLists;
+    PCX_HIP(hipMemsetAsync(unsat_n, 0, sizeof(int32_t), e->stream));
+    PCX_HIP(launch_base_probe(table_of(e), b->d_base, b->d_unsat, unsat_n, dom_of(e), e->stream));
+    int32_t ctl[kDiffLists + 1];
+    pcx_status st = read_small(b, b->d_seedctl, sizeof(ctl), ctl);
+    if (st != PCX_OK) return st;
+    int64_t n = 0;
+    for (int c = 0; c < kDiffLists; ++c)
+      n = (ctl[c] > b->diff_cap || n < 0) ? -1 : n + ctl[c];   // -1: a sub-list lost entries
+    b->probe_diff = n;
+    b->probe_unsat = ctl[kDiffLists];
+    b->probe_version = e->version;
+    b->probe_valid = true;
+  }
+  if (b->probe_diff < 0) return PCX_OK;
+  const int64_t n_diff = b->probe_diff, n_unsat = b->probe_unsat;
+  const int64_t per_var = 3 * b->table_n / std::max<int64_t>(b->nvars, 1) + 1;   // mean adjacency
+  const int64_t pairs = b->h_off.empty() ? b->n_inst * b->table_n : b->h_off.back();
+  if ((n_diff * per_var + n_unsat * b->n_inst) * 16 > pairs) return PCX_OK;
+  *plan = SeedPlan{true, n_diff, n_unsat};
+  return PCX_OK;
+}
+
+// Whether this run goes to the event-driven LDS kernel (launch_local): stores
+// and tables that fit a workgroup's LDS, runs to the fixpoint, and -- outside
+// the persistent mode, which is this kernel or its full-sweep form -- no
+// setting that shapes the other sweeps.  Seeded runs are left to the drain,
+// which touches a fraction of the stores.  Bitset batches keep the sweeps
+// outside the persistent mode: their networks settle in few rounds of costly
+// evaluations, which one compute unit spreads over too few lanes (a 4,000-word,
+// 16,000-propagator store took 0.79 ms here and 0.34 ms in full sweeps).  The
+// limit on the table is where a batch's dense rounds would outlast sweeps by
+// the whole device; a batch of 8 stores of 16,000 variables (64,000 propagators)
+// takes 2.0 ms here and 6.4 ms in batched sweeps.
+constexpr int64_t kLocalBatchProps = (int64_t)1 << 17;
+bool local_wanted(const pcx_batch* b, int32_t mode, bool seeded) {
+  const pcx_config& c = b->e->cfg;
+  if (mode == PCX_MODE_PLAIN) return b->n_inst == 1 && b->h_off.empty() && !b->seeded &&
+                                     pcx_internal::single_local(b->e, b->nvars);
+  if (c.lds_mode == 0 || c.max_sweeps > 0 || c.event_driven == 0 || 3 * b->table_n >= ((int64_t)1 << 31) ||
+      !local_fits(c.device, b->nvars, b->table_n))
+    return false;
+  if (mode == PCX_MODE_PERSISTENT) return true;
+  return mode == PCX_MODE_BATCHED && c.domain == PCX_DOMAIN_INTERVAL && c.event_driven < 0 &&
+         c.props_per_wave == 0 && c.lockstep < 0 && c.mark_queue < 0 && !seeded && !b->seeded &&
+         b->table_n <= kLocalBatchProps;
+}
+
+pcx_status prepare_run(pcx_batch* b, int32_t mode, SeedPlan* plan, bool* local) {
   pcx_engine* e = b->e;
   if ((int64_t)e->op.size() != b->table_n)
     return fail_with(PCX_EINVAL, "table changed since the batch was created");
@@ -450,9 +578,46 @@ pcx_status prepare_run(pcx_batch* b, int32_t mode) {
   b->trail_valid = false;                   // until a drained run from the image lists its changes
   pcx_status st = ensure_pinned(b);
   if (st != PCX_OK) return st;
+  *plan = SeedPlan{};
+  if (mode == PCX_MODE_BATCHED) st = plan_seed(b, plan);
+  if (st != PCX_OK) return st;
+  *local = local_wanted(b, mode, plan->seeded);
+  if (*local) {                             // neither per-instance tables nor mark planes
+    b->seeded = b->seeded_run = false;
+    b->events = true;                       // evaluations are counted: one full sweep, then marks
+    st = ensure_adj_records(e);
+    return st == PCX_OK ? ensure_members(b) : st;
+  }
   st = prepare_tables(b);
   if (st != PCX_OK) return st;
   return prepare_events(b, mode);
+}
+
+// The LDS kernel over the batch: one launch, one workgroup per instance.
+pcx_status run_local(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
+  pcx_engine* e = b->e;
+  SweepTimer tm{b, e->cfg.timing != 0};
+  pcx_status ts = tm.begin(e->stream);
+  if (ts != PCX_OK) return ts;
+  LocalJob job{};
+  job.store = b->d_store;
+  job.nvars = b->nvars;
+  job.n_inst = (int32_t)b->n_inst;
+  job.flags = b->d_flags;
+  job.order = b->d_order;
+  job.queue = b->d_ctl + 3;                 // zeroed with the flags
+  job.tight = b->d_tight;
+  job.adj_off = e->d_adj_off;
+  job.adj_vars = (int32_t)e->adj_vars;
+  job.adj = e->d_adj_rec;
+  job.member = b->h_off.empty() ? nullptr : b->d_member;
+  job.words = bitmap_words(b);
+  PCX_HIP(launch_local(table_of(e), job, dom_of(e), e->cfg.device,
+                       pcx_internal::device_cus(e->cfg.device), e->stream));
+  ts = tm.end(e->stream, true);
+  if (ts != PCX_OK) return ts;
+  std::vector<InstFlags> flags;
+  return collect(b, flags, results, stats, tm);
 }
 
 // Queue planes of a batch (queued marked sweeps), allocated on first use:
@@ -660,62 +825,11 @@ pcx_status ensure_shadow(pcx_batch* b, int gi) {
 // (turn, queue pass) launches replayed as one graph until a turn finds no
 // marks, or finds a plane that lost marks, from which sweep on the bitmap
 // sweeps take over.
-// A run that starts from the loaded stores, whose load listed the values that
-// differ from the base store (the values instances 0-2 agree on), needs in
-// its first sweep only (a) the member propagators adjacent to a listed value
-// of their instance and (b) the propagators the base store does not satisfy,
-// in every instance that holds them: any other propagator reads in instance
-// k the values it reads in the base store, where it tightens nothing.  These are seeded as the first
-// sweep's marks, which makes that sweep a marked sweep, when their count is
-// under 1/16 of the pairs a full sweep evaluates (and the list is complete).
-// This decides; the run launches the seeding (*n_unsat propagators listed
-// in d_unsat) with its own event set.
-pcx_status plan_seed(pcx_batch* b, bool* seeded, int64_t* n_diff_out, int64_t* n_unsat_out) {
-  *seeded = false;
-  *n_diff_out = 0;
-  *n_unsat_out = 0;
+pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, pcx_stats* stats) {
   pcx_engine* e = b->e;
-  if (!b->events || b->seeded_run || !b->run_from_image || !b->diffs_listed || e->cfg.base_seed == 0 ||
-      b->table_n == 0)
-    return PCX_OK;
-  // The probe and the counts depend on the image and the table only: runs
-  // from the same image (after resets) reuse them.
-  if (!b->probe_valid || b->probe_version != e->version) {
-    if (!b->d_unsat) PCX_HIP(hipMalloc(&b->d_unsat, b->table_n * sizeof(int32_t)));
-    int32_t* unsat_n = b->d_seedctl + kDiffLists;
-    PCX_HIP(hipMemsetAsync(unsat_n, 0, sizeof(int32_t), e->stream));
-    PCX_HIP(launch_base_probe(table_of(e), b->d_base, b->d_unsat, unsat_n, dom_of(e), e->stream));
-    int32_t ctl[kDiffLists + 1];
-    pcx_status st = read_small(b, b->d_seedctl, sizeof(ctl), ctl);
-    if (st != PCX_OK) return st;
-    int64_t n = 0;
-    for (int c = 0; c < kDiffLists; ++c)
-      n = (ctl[c] > b->diff_cap || n < 0) ? -1 : n + ctl[c];   // -1: a sub-list lost entries
-    b->probe_diff = n;
-    b->probe_unsat = ctl[kDiffLists];
-    b->probe_version = e->version;
-    b->probe_valid = true;
-  }
-  if (b->probe_diff < 0) return PCX_OK;
-  const int64_t n_diff = b->probe_diff, n_unsat = b->probe_unsat;
-  const int64_t per_var = 3 * b->table_n / std::max<int64_t>(b->nvars, 1) + 1;   // mean adjacency
-  const int64_t pairs = b->h_off.empty() ? b->n_inst * b->table_n : b->h_off.back();
-  if ((n_diff * per_var + n_unsat * b->n_inst) * 16 > pairs) return PCX_OK;
-  *seeded = true;
-  *n_unsat_out = n_unsat;
-  *n_diff_out = n_diff;
-  return PCX_OK;
-}
-
-pcx_status run_batched(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
-  pcx_engine* e = b->e;
-  bool base_seeded = false;
-  int64_t n_diff = 0, n_unsat = 0;
-  {
-    pcx_status ss = plan_seed(b, &base_seeded, &n_diff, &n_unsat);
-    if (ss != PCX_OK) return ss;
-    if (base_seeded) b->seeded_run = true;
-  }
+  const bool base_seeded = plan.seeded && b->events && !b->seeded_run;
+  const int64_t n_diff = plan.n_diff, n_unsat = plan.n_unsat;
+  if (base_seeded) b->seeded_run = true;
   const int ppw = ppw_of(e);
   const int gi = lockstep_of(b);
   SweepTimer tm{b, e->cfg.timing != 0};
@@ -1024,6 +1138,8 @@ void pcx_destroy(pcx_engine* e) {
   (void)hipSetDevice(e->cfg.device);
   if (e->scratch) pcx_batch_destroy(e->scratch);
   dfree(e->d_xo); dfree(e->d_y); dfree(e->d_z); dfree(e->d_adj_off); dfree(e->d_adj);
+  dfree(e->d_adj_rec);
+  if (e->h_io) (void)hipHostFree(e->h_io);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
 }
@@ -1502,12 +1618,14 @@ pcx_status pcx_batch_run(pcx_batch* b, int32_t mode, pcx_result* results, pcx_st
   pcx_engine* e = b->e;
   PCX_HIP(hipSetDevice(e->cfg.device));
   const double t0 = now_ms();
-  pcx_status s = prepare_run(b, mode);
+  SeedPlan plan;
+  bool local = false;
+  pcx_status s = prepare_run(b, mode, &plan, &local);
   if (s != PCX_OK) return s;
   switch (mode) {
-    case PCX_MODE_PLAIN: s = run_plain(b, results, stats); break;
-    case PCX_MODE_BATCHED: s = run_batched(b, results, stats); break;
-    case PCX_MODE_PERSISTENT: s = run_persistent(b, results, stats); break;
+    case PCX_MODE_PLAIN: s = local ? run_local(b, results, stats) : run_plain(b, results, stats); break;
+    case PCX_MODE_BATCHED: s = local ? run_local(b, results, stats) : run_batched(b, plan, results, stats); break;
+    case PCX_MODE_PERSISTENT: s = local ? run_local(b, results, stats) : run_persistent(b, results, stats); break;
     default: return fail_with(PCX_EINVAL, "unknown mode");
   }
   if (stats) stats->wall_ms = now_ms() - t0;
@@ -1768,11 +1886,42 @@ pcx_status pcx_batch_autotune(pcx_batch* b, int32_t reps, pcx_tuning* best, pcx_
   return s;
 }
 
+namespace {
+// A small store through the LDS kernel: the kernel reads and writes the bounds
+// in pinned host memory itself (at most 2 x 160 KB), so a call is two host
+// copies, one launch and one wait.
+pcx_status fixpoint_local(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx_result* out) {
+  PCX_HIP(hipSetDevice(e->cfg.device));
+  pcx_status s = sync_table(e);
+  if (s == PCX_OK) s = ensure_adj_records(e);
+  if (s != PCX_OK) return s;
+  if (e->io_vars < nvars) {
+    if (e->h_io) (void)hipHostFree(e->h_io);
+    e->h_io = nullptr;
+    e->io_vars = 0;
+    PCX_HIP(hipHostMalloc(reinterpret_cast<void**>(&e->h_io), sizeof(InstFlags) + 2 * nvars * sizeof(int32_t)));
+    e->io_vars = nvars;
+  }
+  InstFlags* flags = reinterpret_cast<InstFlags*>(e->h_io);
+  int32_t* plb = reinterpret_cast<int32_t*>(flags + 1);
+  int32_t* pub = plb + nvars;
+  std::memcpy(plb, lb, nvars * sizeof(int32_t));
+  std::memcpy(pub, ub, nvars * sizeof(int32_t));
+  PCX_HIP(pcx_internal::launch_single(e, plb, pub, nvars, flags));
+  PCX_HIP(hipStreamSynchronize(e->stream));
+  std::memcpy(lb, plb, nvars * sizeof(int32_t));
+  std::memcpy(ub, pub, nvars * sizeof(int32_t));
+  if (out) *out = pcx_internal::single_result(e, *flags);
+  return PCX_OK;
+}
+}  // namespace
+
 pcx_status pcx_fixpoint(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx_result* out) {
   if (!e || !lb || !ub) return fail_with(PCX_EINVAL, "NULL argument");
   if (e->cfg.domain != PCX_DOMAIN_INTERVAL) return fail_with(PCX_EINVAL, "pcx_fixpoint needs an interval engine");
   if (nvars <= 0) return fail_with(PCX_EINVAL, "nvars must be positive");
   if (e->max_var >= nvars) return fail_with(PCX_EINVAL, "a propagator names a variable outside the store");
+  if (pcx_internal::single_local(e, nvars)) return fixpoint_local(e, lb, ub, nvars, out);
   if (!e->scratch || e->scratch_nvars != nvars || e->scratch_table != (int64_t)e->op.size()) {
     if (e->scratch) pcx_batch_destroy(e->scratch);
     e->scratch = nullptr;

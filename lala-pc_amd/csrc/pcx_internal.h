@@ -19,13 +19,18 @@ struct pcx_engine {
   int32_t* d_adj_off = nullptr;
   int32_t* d_adj = nullptr;
   uint64_t adj_version = 0;
-  int64_t adj_vars = 0;
+  int64_t adj_vars = 0;               // variables with offsets (max_var + 1 then)
+  int64_t adj_n = 0;                  // adjacency entries
+  int4* d_adj_rec = nullptr;          // the adjacency with table entries (LDS kernel), on demand
+  uint64_t adj_rec_version = 0;
   uint32_t* d_xo = nullptr;
   int32_t* d_y = nullptr;
   int32_t* d_z = nullptr;
   int64_t d_cap = 0;
   hipStream_t stream = nullptr;
   pcx_batch* scratch = nullptr;       // batch of one for pcx_fixpoint / pcx_ask_all
+  uint8_t* h_io = nullptr;            // pinned: flags and bounds of a small pcx_fixpoint
+  int64_t io_vars = 0;                // room of h_io
   int64_t scratch_nvars = -1;
   int64_t scratch_table = -1;
 };
@@ -134,6 +139,11 @@ pcx_status sync_table(pcx_engine* e);   // upload the table if it changed
 int dom_of(const pcx_engine* e);        // kernel domain for this engine
 int device_cus(int device);             // compute units of a device
 pcx_status ensure_adjacency(pcx_engine* e);   // variable -> table positions, on the device
+pcx_status ensure_adj_records(pcx_engine* e); // the same with each propagator's table entry
+// one small store through the LDS kernel (see pcx_engine.hip)
+bool single_local(const pcx_engine* e, int64_t nvars);
+hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx::InstFlags* flags);
+pcx_result single_result(const pcx_engine* e, const pcx::InstFlags& f);
 }  // namespace pcx_internal
 
 #define PCX_HIP(call)                                                                  \

@@ -304,6 +304,34 @@ hipError_t launch_persistent(const Table& t, int2* store, int64_t nvars, const S
                              int32_t n_inst, int32_t* queue, unsigned long long* tight,
                              int32_t max_sweeps, int dom, int grid, bool lds, int64_t lds_cap,
                              hipStream_t st);
+// Event-driven fixpoints of stores that fit in a workgroup's LDS, one
+// workgroup per instance (pcx_local.hip).  Instances come either from a
+// batch's stores (store, n_inst slices; flags already initialised, an instance
+// with failed_at set is left alone; taken in `order` from *queue, zeroed by
+// the caller) or from one pair of bound arrays (lb / ub, one instance, which
+// the kernel reads and writes in place: memory the device can address,
+// emptiness found by the kernel, flags written whole).
+struct LocalJob {
+  int32_t* lb;              // or nullptr
+  int32_t* ub;
+  int2* store;              // or nullptr
+  int64_t nvars;
+  int32_t n_inst;
+  InstFlags* flags;         // [n_inst]
+  const int32_t* order;     // [n_inst], or nullptr: in index order
+  int32_t* queue;           // [1], or nullptr (one instance)
+  unsigned long long* tight;// [2 * kTightSlots] (round 0, later rounds), or nullptr
+  const int32_t* adj_off;   // [adj_vars + 1]
+  int32_t adj_vars;         // variables the table names, at most nvars
+  const int4* adj;          // adjacency records (launch_adj_records)
+  const uint32_t* member;   // [n_inst * words], or nullptr: every propagator
+  int64_t words;
+};
+// whether a store and a table fit (store, bitmaps and lists in LDS)
+bool local_fits(int device, int64_t nvars, int64_t n_props);
+hipError_t launch_local(const Table& t, const LocalJob& job, int dom, int device, int cus, hipStream_t st);
+// rec[i] = {adj[i], xo, y, z of that propagator} for n adjacency entries
+hipError_t launch_adj_records(const Table& t, const int32_t* adj, int64_t n, int4* rec, hipStream_t st);
 // resident workgroups per CU (lds_bytes of dynamic LDS per workgroup)
 int persistent_blocks_per_cu(int dom, int64_t lds_bytes);
 // empty (may be nullptr): per-instance bytes, 1 = the store starts empty

@@ -15,84 +15,16 @@
 //   kBits    bitset store
 #include "pcx_kernels.h"
 #include "../../include/pcx_model.h"
-#include "pcx_prop.h"
+#include "pcx_device.h"
 
 #include <type_traits>
 
 namespace pcx {
 
-__device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
-
-// Values the whole wave agrees on (work-item indices, descriptors read
-// through them) moved to scalar registers: the compiler cannot prove a load
-// from a uniform address returns a uniform value, and would otherwise keep
-// them, and everything derived from them, in VGPRs.
-__device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t uni(int64_t v) {
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)(uint32_t)v);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int32_t)(uint32_t)((uint64_t)v >> 32));
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-template <class T>
-__device__ __forceinline__ T* uni(T* p) { return reinterpret_cast<T*>(uni((int64_t)(uintptr_t)p)); }
-
 // Subset indices are read once per sweep: stream them past the caches so
 // they do not evict the store and table lines that are reused.
 __device__ __forceinline__ int64_t prop_at(const int32_t* __restrict__ idx, int64_t q) {
   return idx ? (int64_t)__builtin_nontemporal_load(idx + q) : q;
-}
-
-__device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
-  return v;
-}
-
-// ---- store access policies ------------------------------------------------
-// Agent scope (sweep kernels: ordered by kernel boundaries) or workgroup
-// scope (persistent kernel: one workgroup owns an instance).
-template <int SCOPE>
-__device__ __forceinline__ u64 load_word(const void* p) {
-  if constexpr (SCOPE == __HIP_MEMORY_SCOPE_AGENT) return *reinterpret_cast<const u64*>(p);
-  else return __hip_atomic_load(reinterpret_cast<const u64*>(p), __ATOMIC_RELAXED, SCOPE);
-}
-__device__ __forceinline__ int2 as_itv(u64 v) {
-  return make_int2((int32_t)(uint32_t)v, (int32_t)(uint32_t)(v >> 32));
-}
-__device__ __forceinline__ u64 itv_bits(int2 v) { return (u64)(uint32_t)v.x | ((u64)(uint32_t)v.y << 32); }
-
-// Meet interval `n` into variable v, whose value was read as `cur`.
-// Returns true when this call tightened a bound of v.
-template <int SCOPE>
-__device__ __forceinline__ bool meet_itv(int2* __restrict__ st, int32_t v, int2 cur, int2 n,
-                                         bool& chg, bool& fail, int& nt) {
-  bool t = false;
-  if (n.x > cur.x) {
-    const int old = __hip_atomic_fetch_max(&st[v].x, n.x, __ATOMIC_RELAXED, SCOPE);
-    if (old < n.x) { t = true; ++nt; }
-    if (n.x > cur.y) fail = true;          // cur.y >= current ub
-  }
-  if (n.y < cur.y) {
-    const int old = __hip_atomic_fetch_min(&st[v].y, n.y, __ATOMIC_RELAXED, SCOPE);
-    if (old > n.y) { t = true; ++nt; }
-    if (n.y < cur.x) fail = true;
-  }
-  chg |= t;
-  return t;
-}
-
-// AND mask `n` into word v, whose value was read as `cur`.
-template <int SCOPE>
-__device__ __forceinline__ bool meet_word(u64* __restrict__ st, int32_t v, u64 cur, u64 n,
-                                          bool& chg, bool& fail, int& nt) {
-  bool t = false;
-  if ((cur & n) != cur) {
-    const u64 old = __hip_atomic_fetch_and(&st[v], n, __ATOMIC_RELAXED, SCOPE);
-    if ((old & n) != old) { t = true; ++nt; }
-    if ((old & n) == 0) fail = true;       // the word is now empty
-  }
-  chg |= t;
-  return t;
 }
 
 // Where a tightening of variable v is recorded for the next sweep of one

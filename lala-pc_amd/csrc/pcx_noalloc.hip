@@ -105,6 +105,17 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   hipStream_t s = e->stream;
   const int dom = pcx_internal::dom_of(e);
 
+  // A small store whose adjacency records an earlier pcx_fixpoint built: one
+  // launch on the caller's arrays, the flags read back after it.
+  if (pcx_internal::single_local(e, nvars) && e->d_adj_rec && e->adj_rec_version == e->version) {
+    InstFlags f{};
+    PCX_HIP(pcx_internal::launch_single(e, d_lb, d_ub, nvars, d_flags));
+    PCX_HIP(hipMemcpyAsync(&f, d_flags, sizeof(f), hipMemcpyDeviceToHost, s));
+    PCX_HIP(hipStreamSynchronize(s));
+    if (out) *out = pcx_internal::single_result(e, f);
+    return PCX_OK;
+  }
+
   // Every value the sweeps read is written first: flags, counters, store.
   const WorkList wl = worklist_of(d_act, d_base, d_ctl);
   PCX_HIP(launch_init_flags(d_flags, 1, wl, s));

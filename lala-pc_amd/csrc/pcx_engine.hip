@@ -128,11 +128,12 @@ pcx_status ensure_adjacency(pcx_engine* e) {
   return PCX_OK;
 }
 
-// One store through the LDS kernel: up to 48 K propagators, where one workgroup
-// still beats sweeps by the whole device (ms per fixpoint at 1,000 / 16,000 /
-// 48,000 / 74,000 propagators: 0.23 / 0.66 / 1.4 / 1.9 here, 0.95 / 1.9 / 2.0 /
-// 1.6 in sweeps).  Intervals, automatic settings and runs to the fixpoint only.
-constexpr int64_t kLocalSingleProps = 48 * 1024;
+// One store through the LDS kernel: up to 16 K propagators, where one workgroup
+// still beats sweeps by the whole device, which chase too (us per fixpoint at
+// 1,000 / 8,000 / 16,000 / 24,000 / 48,000 propagators: 156 / 409 / 562 / 673 /
+// 1,293 here, 301 / 568 / 590 / 596 / 668 there).  Intervals, automatic settings
+// and runs to the fixpoint only.
+constexpr int64_t kLocalSingleProps = 16 * 1024;
 bool single_local(const pcx_engine* e, int64_t nvars) {
   const pcx_config& c = e->cfg;
   const int64_t n = (int64_t)e->op.size();
@@ -167,6 +168,20 @@ pcx_result single_result(const pcx_engine* e, const InstFlags& f) {
   r.sweeps = r.failed ? (int64_t)f.failed_at + 1 : (int64_t)last + 2;
   r.evals = f.failed_at == -1 ? 0 : (int64_t)e->op.size() + f.marked_evals;
   return r;
+}
+
+// Whether plain runs of one interval store chase (launch_sweep_chase): automatic
+// settings, runs to the fixpoint, and the adjacency records there or room for
+// them (a quarter of free memory).
+bool chase_wanted(const pcx_engine* e) {
+  const pcx_config& c = e->cfg;
+  const int64_t n = (int64_t)e->op.size();
+  if (c.domain != PCX_DOMAIN_INTERVAL || c.max_sweeps > 0 || c.event_driven >= 0 || c.props_per_wave != 0 ||
+      c.mark_queue >= 0 || n == 0 || 3 * n >= ((int64_t)1 << 31))
+    return false;
+  if (e->d_adj_rec && e->adj_rec_version == e->version) return true;
+  size_t free_b = 0, total_b = 0;
+  return hipMemGetInfo(&free_b, &total_b) == hipSuccess && 3 * (uint64_t)n * sizeof(int4) <= free_b / 4;
 }
 
 // 16 B per adjacency entry, written by the device from the table it holds.
@@ -304,7 +319,7 @@ pcx_status collect(pcx_batch* b, std::vector<InstFlags>& flags, pcx_result* resu
       r.evals = first + f.marked_evals;
       full_evals += first;
     } else {
-      r.evals = r.sweeps * inst_size(b, k);
+      r.evals = r.sweeps * inst_size(b, k) + f.marked_evals;   // (evaluations of chases)
       full_evals += r.evals;
     }
     evals += r.evals;
@@ -588,6 +603,12 @@ pcx_status prepare_run(pcx_batch* b, int32_t mode, SeedPlan* plan, bool* local) 
     st = ensure_adj_records(e);
     return st == PCX_OK ? ensure_members(b) : st;
   }
+  b->chase = mode == PCX_MODE_PLAIN && !b->seeded && b->n_inst == 1 && b->h_off.empty() &&
+             pcx_internal::chase_wanted(e);
+  if (b->chase) {                           // full sweeps that chase: no marks are kept
+    b->events = b->seeded_run = false;
+    return ensure_adj_records(e);
+  }
   st = prepare_tables(b);
   if (st != PCX_OK) return st;
   return prepare_events(b, mode);
@@ -737,7 +758,8 @@ pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
     for (; !done;) {
       // Full sweeps are timed one by one; consecutive marked sweeps as one span.
       int n_marked = 0;
-      for (int g = 0; g < group; ++g, ++s) {
+      const int count = b->chase ? (s == 0 ? pcx_internal::kChaseAfter + 2 : 2) : group;
+      for (int g = 0; g < count; ++g, ++s) {
         if (e->cfg.max_sweeps > 0 && s >= e->cfg.max_sweeps) break;
         const bool marked = b->events && (s > 0 || b->seeded_run);
         pcx_status ts = PCX_OK;
@@ -748,8 +770,12 @@ pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
                                             e->stream));
           ++n_marked;
         } else {
-          PCX_HIP(launch_sweep_plain(tk, st, idx, m, s, f, b->d_tight, ppw, dom_of(e), b->stream,
-                                     e->stream, b->events ? &ev : nullptr, k));
+          if (b->chase && s >= pcx_internal::kChaseAfter)
+            PCX_HIP(launch_sweep_chase(tk, st, s, f, b->d_tight, e->d_adj_off, e->d_adj_rec, dom_of(e),
+                                       pcx_internal::device_cus(e->cfg.device), e->stream));
+          else
+            PCX_HIP(launch_sweep_plain(tk, st, idx, m, s, f, b->d_tight, ppw, dom_of(e), b->stream,
+                                       e->stream, b->events ? &ev : nullptr, k));
           ts = tm.end(e->stream, true);
           if (ts != PCX_OK) return ts;
         }

@@ -71,6 +71,7 @@ struct pcx_batch {
   bool events = false;                // this run uses marked-only sweeps
   bool seeded = false;                // the next run may start from seeded marks
   bool seeded_run = false;            // this run starts with a marked sweep
+  bool chase = false;                 // this run's sweeps chase what they tighten
   bool marks_clean = false;           // both mark planes and the summaries are zero
   // first sweeps seeded from a base store (per variable the value instances
   // 0-2 agree on): the base, the values of the image that differ from it
@@ -143,6 +144,8 @@ pcx_status ensure_adj_records(pcx_engine* e); // the same with each propagator's
 // one small store through the LDS kernel (see pcx_engine.hip)
 bool single_local(const pcx_engine* e, int64_t nvars);
 hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx::InstFlags* flags);
+bool chase_wanted(const pcx_engine* e);       // plain runs of one store chase
+constexpr int kChaseAfter = 4;                // plain sweeps before the first chase (see pcx_chase.hip)
 pcx_result single_result(const pcx_engine* e, const pcx::InstFlags& f);
 }  // namespace pcx_internal
 

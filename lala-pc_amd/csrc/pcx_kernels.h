@@ -304,6 +304,11 @@ hipError_t launch_persistent(const Table& t, int2* store, int64_t nvars, const S
                              int32_t n_inst, int32_t* queue, unsigned long long* tight,
                              int32_t max_sweeps, int dom, int grid, bool lds, int64_t lds_cap,
                              hipStream_t st);
+// Full sweep of one interval store whose waves chase what they tighten in the
+// same launch (pcx_chase.hip); adj: the adjacency records, adj_off their ranges.
+hipError_t launch_sweep_chase(const Table& t, int2* store, int32_t sweep, InstFlags* flags,
+                              unsigned long long* tight, const int32_t* adj_off, const int4* adj, int dom, int cus,
+                              hipStream_t st);
 // Event-driven fixpoints of stores that fit in a workgroup's LDS, one
 // workgroup per instance (pcx_local.hip).  Instances come either from a
 // batch's stores (store, n_inst slices; flags already initialised, an instance

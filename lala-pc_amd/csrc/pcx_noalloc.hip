@@ -125,7 +125,10 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   PCX_HIP(launch_store_check_empty(d_store, nvars, 1, d_flags, dom, s));
 
   // Full sweeps, the flags read back every `group` sweeps (as the plain mode
-  // does), until a sweep changed nothing or the store failed.
+  // does), until a sweep changed nothing or the store failed; from the fifth on
+  // they chase what they tighten when an earlier pcx_fixpoint left the adjacency
+  // records.
+  const bool chase = e->d_adj_rec && e->adj_rec_version == e->version && pcx_internal::chase_wanted(e);
   const Table t{e->d_xo, e->d_y, e->d_z, m};
   int ppw = e->cfg.props_per_wave ? std::min(e->cfg.props_per_wave, 512) : 0;
   if (!ppw) {
@@ -139,9 +142,14 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   InstFlags hf{};
   int32_t sw = 0;
   for (;;) {
-    for (int g = 0; g < group; ++g, ++sw) {
+    const int count = chase ? (sw == 0 ? pcx_internal::kChaseAfter + 2 : 2) : group;
+    for (int g = 0; g < count; ++g, ++sw) {
       if (maxs > 0 && sw >= maxs) break;
-      PCX_HIP(launch_sweep_plain(t, d_store, nullptr, m, sw, d_flags, d_tight, ppw, dom, false, s));
+      if (chase && sw >= pcx_internal::kChaseAfter)
+        PCX_HIP(launch_sweep_chase(t, d_store, sw, d_flags, d_tight, e->d_adj_off, e->d_adj_rec, dom,
+                                   pcx_internal::device_cus(e->cfg.device), s));
+      else
+        PCX_HIP(launch_sweep_plain(t, d_store, nullptr, m, sw, d_flags, d_tight, ppw, dom, false, s));
     }
     PCX_HIP(hipMemcpyAsync(&hf, d_flags, sizeof(hf), hipMemcpyDeviceToHost, s));
     PCX_HIP(hipStreamSynchronize(s));
@@ -158,7 +166,7 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
     r.has_changed = last >= 0;
     r.sweeps = r.failed ? (int64_t)hf.failed_at + 1 : (int64_t)last + 2;
     if (maxs > 0 && r.sweeps > maxs) r.sweeps = maxs;
-    r.evals = r.sweeps * m;
+    r.evals = r.sweeps * m + hf.marked_evals;    // (evaluations of chases)
     *out = r;
   }
   return PCX_OK;

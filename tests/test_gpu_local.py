@@ -68,11 +68,11 @@ def _check_batch(pir, lo, hi, V, mode, off=None, idx=None):
     return st, ok
 
 
-@pytest.mark.parametrize("P", [31, 32, 33, 63, 64, 65, 1000, 2048, 12007, 49152])
+@pytest.mark.parametrize("P", [31, 32, 33, 63, 64, 65, 1000, 2048, 12007, 16384, 16385, 49152])
 def test_single_store(gpu, P):
-    """Tables around the bitmap's words and the lists' room, up to the largest
-    that one store takes to this kernel; the told store, one that starts empty
-    and one that fails."""
+    """Tables around the bitmap's words and the lists' room, up to 16,384
+    propagators, the largest that one store takes to this kernel, and beyond; the
+    told store, one that starts empty and one that fails."""
     V = max(80, P // 4 + 1)
     net = pcx.gen_network(pcx.gen_params(seed=P, nvars=V, nprops=P, chain_len=50))
     pir, lb, ub = _told(net)

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "pcx_internal.h"
+#include "pcx_xfer.h"
 #include "../../include/pcx_model.h"
 
 using namespace pcx;
@@ -198,6 +199,7 @@ pcx_status ensure_adj_records(pcx_engine* e) {
 
 }  // namespace pcx_internal
 
+using pcx_internal::copy_to_host;
 using pcx_internal::dom_of;
 using pcx_internal::ensure_adj_records;
 using pcx_internal::ensure_adjacency;
@@ -1155,6 +1157,7 @@ pcx_status pcx_create(const pcx_config* cfg, pcx_engine** out) {
     delete e;
     return fail_with(PCX_EDEVICE, std::string("hipStreamCreate: ") + hipGetErrorString(he));
   }
+  pcx_internal::xfer_acquire();
   *out = e;
   return PCX_OK;
 }
@@ -1168,6 +1171,7 @@ void pcx_destroy(pcx_engine* e) {
   if (e->h_io) (void)hipHostFree(e->h_io);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   delete e;
+  pcx_internal::xfer_release();
 }
 
 pcx_status pcx_tell(pcx_engine* e, const int32_t* op, const int32_t* x, const int32_t* y,
@@ -1633,9 +1637,8 @@ pcx_status pcx_batch_read(pcx_batch* b, int32_t* lb, int32_t* ub) {
   if (!b->d_unpack) PCX_HIP(hipMalloc(&b->d_unpack, 2 * n * sizeof(int32_t)));
   int32_t* d_lb = b->d_unpack;
   PCX_HIP(launch_store_unpack(b->d_store, d_lb, d_lb + n, n, e->stream));
-  PCX_HIP(hipMemcpyAsync(lb, d_lb, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
-  PCX_HIP(hipMemcpyAsync(ub, d_lb + n, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
-  PCX_HIP(hipStreamSynchronize(e->stream));
+  const size_t bytes = n * sizeof(int32_t);
+  PCX_HIP(copy_to_host(lb, bytes, ub, bytes, d_lb, e->cfg.device, e->stream));
   return PCX_OK;
 }
 
@@ -2058,9 +2061,8 @@ pcx_status pcx_bits_batch_read(pcx_batch* b, uint64_t* words) {
   if (b->e->cfg.domain != PCX_DOMAIN_BITSET) return fail_with(PCX_EINVAL, "bitset batch expected");
   pcx_engine* e = b->e;
   PCX_HIP(hipSetDevice(e->cfg.device));
-  PCX_HIP(hipMemcpyAsync(words, b->d_store, b->n_inst * b->nvars * sizeof(uint64_t),
-                         hipMemcpyDeviceToHost, e->stream));
-  PCX_HIP(hipStreamSynchronize(e->stream));
+  PCX_HIP(copy_to_host(words, b->n_inst * b->nvars * sizeof(uint64_t), nullptr, 0, b->d_store, e->cfg.device,
+                       e->stream));
   return PCX_OK;
 }
 

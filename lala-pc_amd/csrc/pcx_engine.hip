@@ -1366,6 +1366,7 @@ void pcx_batch_destroy(pcx_batch* b) {
   if (b->plain_queue_graph) (void)hipGraphExecDestroy(b->plain_queue_graph);
   dfree(b->d_q); dfree(b->d_qctl);
   dfree(b->d_diff); dfree(b->d_diff_val); dfree(b->d_unsat); dfree(b->d_trail); dfree(b->d_trail_n); dfree(b->d_bvar); dfree(b->d_seedctl); dfree(b->d_base); dfree(b->d_base_alt);
+  dfree(b->d_ask);
   for (hipEvent_t ev : b->load_ev)
     if (ev) (void)hipEventDestroy(ev);
   delete b;
@@ -1742,46 +1743,103 @@ bool trees_valid(const int32_t* nodes, int64_t n_nodes, const int64_t* off, int6
 }
 }  // namespace
 
+namespace {
+// Room for an ask's arrays, kept with the batch.
+pcx_status ask_room(pcx_batch* b, int64_t bytes) {
+  if (b->ask_bytes >= bytes) return PCX_OK;
+  dfree(b->d_ask);
+  b->ask_bytes = 0;
+  PCX_HIP(hipMalloc(&b->d_ask, bytes));
+  b->ask_bytes = bytes;
+  return PCX_OK;
+}
+
+// Stores from which on formulas are asked a wave's lanes at a time.
+constexpr int64_t kLanesMin = 16;
+
+// The current stores' interleaved copy in groups of gi; false when there is no
+// memory for it.
+bool interleaved(pcx_batch* b, int gi) {
+  if (b->store_is_image && b->image_in_shadow && b->shadow_gi == gi) return true;   // the load wrote it
+  const int64_t words = (b->n_inst + gi - 1) / gi * gi * b->nvars;
+  if (b->shadow_words < words) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || (uint64_t)words * sizeof(int2) > free_b / 4) return false;
+  }
+  // (a copy that holds the only image is written out before it goes)
+  if (materialize_image(b) != PCX_OK || ensure_shadow(b, gi) != PCX_OK) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (launch_interleave(b->d_store, b->d_shadow, b->nvars, b->n_inst, gi, b->e->stream) != hipSuccess) return false;
+  b->shadow_is_image = b->store_is_image;
+  b->shadow_gi = gi;
+  return true;
+}
+}  // namespace
+
 pcx_status pcx_batch_ask_formulas(pcx_batch* b, const int32_t* nodes, int64_t n_nodes, const int64_t* off,
                                   int64_t n_formulas, int32_t* extractable) {
   if (!b || !off || !extractable || (n_nodes > 0 && !nodes)) return fail_with(PCX_EINVAL, "NULL argument");
   if (n_nodes < 0 || n_formulas < 0) return fail_with(PCX_EINVAL, "negative size");
   pcx_engine* e = b->e;
   if (e->cfg.domain != PCX_DOMAIN_INTERVAL) return fail_with(PCX_EINVAL, "formula trees are asked on interval batches");
-  std::string why;
-  if (!trees_valid(nodes, n_nodes, off, n_formulas, b->nvars, &why)) return fail_with(PCX_EINVAL, "formula trees: " + why);
+  if (off[0] != 0 || off[n_formulas] != n_nodes)
+    return fail_with(PCX_EINVAL, "formula trees: offsets do not cover the nodes");
   PCX_HIP(hipSetDevice(e->cfg.device));
-  int4* d_nodes = nullptr;
-  int64_t* d_off = nullptr;
-  int32_t* d_ok = nullptr;
-  uint8_t* d_empty = nullptr;
-  auto release = [&]() {
-    for (void* p : {(void*)d_nodes, (void*)d_off, (void*)d_ok, (void*)d_empty}) if (p) (void)hipFree(p);
-  };
-  hipError_t he = hipMalloc(&d_nodes, std::max<int64_t>(n_nodes, 1) * sizeof(int4));
-  if (he == hipSuccess) he = hipMalloc(&d_off, (n_formulas + 1) * sizeof(int64_t));
-  if (he == hipSuccess) he = hipMalloc(&d_ok, b->n_inst * sizeof(int32_t));
-  if (he == hipSuccess) he = hipMalloc(&d_empty, b->n_inst);
-  if (he == hipSuccess && n_nodes > 0)
+  pcx_status ps = ensure_pinned(b);
+  if (ps != PCX_OK) return ps;
+  // One buffer for the call's arrays, kept with the batch.
+  auto up = [](int64_t bytes) { return (bytes + 255) & ~(int64_t)255; };
+  const int64_t at_off = up(n_nodes * sizeof(int4)), at_ok = at_off + up((n_formulas + 1) * sizeof(int64_t));
+  const int64_t at_empty = at_ok + up(b->n_inst * sizeof(int32_t)), at_verdict = at_empty + up(b->n_inst);
+  pcx_status ws = ask_room(b, at_verdict + 2 * sizeof(int32_t));
+  if (ws != PCX_OK) return ws;
+  int4* d_nodes = reinterpret_cast<int4*>(b->d_ask);
+  int64_t* d_off = reinterpret_cast<int64_t*>(b->d_ask + at_off);
+  int32_t* d_ok = reinterpret_cast<int32_t*>(b->d_ask + at_ok);
+  uint8_t* d_empty = b->d_ask + at_empty;
+  int32_t* d_verdict = reinterpret_cast<int32_t*>(b->d_ask + at_verdict);
+  hipError_t he = hipSuccess;
+  if (n_nodes > 0)
     he = hipMemcpyAsync(d_nodes, nodes, n_nodes * sizeof(int4), hipMemcpyHostToDevice, e->stream);
   if (he == hipSuccess)
     he = hipMemcpyAsync(d_off, off, (n_formulas + 1) * sizeof(int64_t), hipMemcpyHostToDevice, e->stream);
+  // The trees are checked where they are; one that is not well formed is looked
+  // up again on the host for the message, and none is asked.
+  if (he == hipSuccess) he = hipMemsetAsync(d_verdict, 0, 2 * sizeof(int32_t), e->stream);
+  if (he == hipSuccess)
+    he = launch_trees_check(d_nodes, n_nodes, d_off, n_formulas, b->nvars, d_verdict, e->stream);
+  int32_t verdict[2] = {0, 0};
+  if (he == hipSuccess) {
+    ps = read_small(b, d_verdict, sizeof(verdict), verdict);
+    if (ps != PCX_OK) return ps;
+    if (verdict[0]) {
+      std::string why;
+      if (trees_valid(nodes, n_nodes, off, n_formulas, b->nvars, &why)) why = "refused on the device";
+      return fail_with(PCX_EINVAL, "formula trees: " + why);
+    }
+  }
+  const int depth = std::max(verdict[1], 1);
   std::vector<int32_t> ones(b->n_inst, 1);
   if (he == hipSuccess)
     he = hipMemcpyAsync(d_ok, ones.data(), b->n_inst * sizeof(int32_t), hipMemcpyHostToDevice, e->stream);
   if (he == hipSuccess) he = hipMemsetAsync(d_empty, 0, b->n_inst, e->stream);
   if (he == hipSuccess)
     he = launch_store_empty_map(b->d_store, b->nvars, (int32_t)b->n_inst, d_empty, dom_of(e), e->stream);
-  if (he == hipSuccess)
+  // Enough stores for a wave's lanes: over the interleaved copy.
+  if (he == hipSuccess && b->n_inst >= kLanesMin && interleaved(b, kWave))
+    he = launch_formula_lanes(d_nodes, d_off, n_formulas, depth, b->d_shadow, b->nvars, b->n_inst, d_ok,
+                              pcx_internal::device_cus(e->cfg.device), e->stream);
+  else if (he == hipSuccess)
     he = launch_formula_ask(d_nodes, d_off, n_formulas, b->d_store, b->nvars, b->n_inst, d_ok, e->stream);
   std::vector<uint8_t> empty(b->n_inst);
   if (he == hipSuccess)
     he = hipMemcpyAsync(extractable, d_ok, b->n_inst * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
   if (he == hipSuccess)
     he = hipMemcpyAsync(empty.data(), d_empty, b->n_inst, hipMemcpyDeviceToHost, e->stream);
-  if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-  else (void)hipStreamSynchronize(e->stream);     // nothing queued still uses the buffers
-  release();
+  const hipError_t se = hipStreamSynchronize(e->stream);      // nothing queued still uses the host arrays
+  if (he == hipSuccess) he = se;
   if (he != hipSuccess) return fail_with(PCX_EDEVICE, std::string("formula ask: ") + hipGetErrorString(he));
   for (int64_t k = 0; k < b->n_inst; ++k) extractable[k] = extractable[k] && !empty[k];
   return PCX_OK;

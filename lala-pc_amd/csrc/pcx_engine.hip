@@ -1744,7 +1744,9 @@ bool trees_valid(const int32_t* nodes, int64_t n_nodes, const int64_t* off, int6
 }  // namespace
 
 namespace {
-// Room for an ask's arrays, kept with the batch.
+// Room for an ask's arrays, kept with the batch (the positions of pcx_batch_ask up
+// to kAskKeep bytes).
+constexpr int64_t kAskKeep = (int64_t)64 << 20;
 pcx_status ask_room(pcx_batch* b, int64_t bytes) {
   if (b->ask_bytes >= bytes) return PCX_OK;
   dfree(b->d_ask);
@@ -1859,48 +1861,52 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   const int64_t n = b->n_inst;
   const Table t = table_of(e);
   const Subsets sub{b->h_off.empty() ? nullptr : b->d_off, b->d_idx};
-  int64_t* d_live = nullptr;
-  int32_t* d_empty = nullptr;
-  int64_t* d_off = nullptr;
-  int32_t* d_out = nullptr;
-  auto release = [&]() { dfree(d_live); dfree(d_empty); dfree(d_off); dfree(d_out); };
-  std::vector<int64_t> live(n);
-  std::vector<int32_t> empty(n);
-  hipError_t he = hipMalloc(&d_live, n * sizeof(int64_t));
-  if (he == hipSuccess) he = hipMalloc(&d_empty, n * sizeof(int32_t));
-  if (he == hipSuccess)
-    he = launch_batch_ask(t, b->d_store, b->nvars, sub, b->table_n, n, d_live, d_empty, nullptr, nullptr,
-                          e->stream);
-  if (he == hipSuccess) he = hipMemcpyAsync(live.data(), d_live, n * sizeof(int64_t), hipMemcpyDeviceToHost, e->stream);
-  if (he == hipSuccess) he = hipMemcpyAsync(empty.data(), d_empty, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
-  if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-  if (he != hipSuccess) {
-    release();
-    return fail_with(PCX_EDEVICE, std::string("batch ask: ") + hipGetErrorString(he));
-  }
+  // One buffer for the call's arrays, kept with the batch; the positions' too
+  // while they are few.
+  int64_t most = b->h_off.empty() ? b->table_n : 0;
+  for (int64_t k = 0; k < n && !b->h_off.empty(); ++k) most = std::max(most, inst_size(b, k));
+  const int64_t chunks = ask_chunks(most), cells = n * chunks;
+  auto up = [](int64_t bytes) { return (bytes + 255) & ~(int64_t)255; };
+  const int64_t at_count = up(cells * (kAskChunk / 8)), at_place = at_count + up(cells * sizeof(int32_t));
+  const int64_t at_off = at_place + up(cells * sizeof(int64_t)), at_empty = at_off + up((n + 1) * sizeof(int64_t));
+  const int64_t at_out = at_empty + up(n * sizeof(int32_t));
+  const int64_t pairs = b->h_off.empty() ? n * b->table_n : b->h_off.back();
+  const int64_t room = live_idx ? std::max<int64_t>(0, std::min(cap, pairs)) : 0;
+  const bool kept = room * (int64_t)sizeof(int32_t) <= kAskKeep;
+  st = ask_room(b, at_out + (kept ? room * sizeof(int32_t) : 0));
+  if (st != PCX_OK) return st;
+  AskWork w{};
+  w.bits = reinterpret_cast<unsigned long long*>(b->d_ask);
+  w.count = reinterpret_cast<int32_t*>(b->d_ask + at_count);
+  w.place = reinterpret_cast<int64_t*>(b->d_ask + at_place);
+  w.off = reinterpret_cast<int64_t*>(b->d_ask + at_off);
+  w.empty = reinterpret_cast<int32_t*>(b->d_ask + at_empty);
+  int32_t* d_big = nullptr;
+  if (!kept) PCX_HIP(hipMalloc(&d_big, room * sizeof(int32_t)));
+  int32_t* const d_out = kept ? reinterpret_cast<int32_t*>(b->d_ask + at_out) : d_big;
   std::vector<int64_t> off(n + 1, 0);
-  for (int64_t k = 0; k < n; ++k) off[k + 1] = off[k] + live[k];
-  if (extractable)
-    for (int64_t k = 0; k < n; ++k) extractable[k] = !empty[k] && live[k] == 0;
-  if (live_off) std::copy(off.begin(), off.end(), live_off);
-  if (live_idx) {
-    if (off[n] > cap) {
-      release();
-      return fail_with(PCX_EINVAL, "live_idx capacity too small (live_off[n_inst] holds the size needed)");
-    }
-    if (off[n] > 0) {
-      he = hipMalloc(&d_off, (n + 1) * sizeof(int64_t));
-      if (he == hipSuccess) he = hipMalloc(&d_out, off[n] * sizeof(int32_t));
-      if (he == hipSuccess) he = hipMemcpyAsync(d_off, off.data(), (n + 1) * sizeof(int64_t), hipMemcpyHostToDevice, e->stream);
-      if (he == hipSuccess)
-        he = launch_batch_ask(t, b->d_store, b->nvars, sub, b->table_n, n, nullptr, nullptr, d_off, d_out,
-                              e->stream);
-      if (he == hipSuccess) he = hipMemcpyAsync(live_idx, d_out, off[n] * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
-      if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
-    }
-  }
-  release();
+  std::vector<int32_t> empty(n);
+  hipError_t he = hipMemsetAsync(w.empty, 0, n * sizeof(int32_t), e->stream);
+  if (he == hipSuccess)
+    he = launch_ask_bits(t, b->d_store, b->nvars, sub, b->table_n, n, chunks, w, e->cfg.device,
+                         pcx_internal::device_cus(e->cfg.device), e->stream);
+  if (he == hipSuccess) he = launch_ask_write(sub, n, chunks, w, d_out, room, e->stream);
+  if (he == hipSuccess)
+    he = hipMemcpyAsync(off.data(), w.off, (n + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, e->stream);
+  if (he == hipSuccess && extractable)
+    he = hipMemcpyAsync(empty.data(), w.empty, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
+  const hipError_t se = hipStreamSynchronize(e->stream);
+  if (he == hipSuccess) he = se;
+  const bool fits = !live_idx || off[n] <= cap;
+  if (he == hipSuccess && fits && live_idx && off[n] > 0)
+    he = copy_to_host(live_idx, off[n] * sizeof(int32_t), nullptr, 0, d_out, e->cfg.device, e->stream);
+  if (d_big) (void)hipFree(d_big);
   if (he != hipSuccess) return fail_with(PCX_EDEVICE, std::string("batch ask: ") + hipGetErrorString(he));
+  if (extractable)
+    for (int64_t k = 0; k < n; ++k) extractable[k] = !empty[k] && off[k + 1] == off[k];
+  if (live_off) std::copy(off.begin(), off.end(), live_off);
+  if (!fits)
+    return fail_with(PCX_EINVAL, "live_idx capacity too small (live_off[n_inst] holds the size needed)");
   return PCX_OK;
 }
 

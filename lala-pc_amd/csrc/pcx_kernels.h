@@ -360,12 +360,23 @@ hipError_t launch_burst_slots(const SlotDesc* slots, InstFlags* flags, int32_t n
                               hipStream_t st);
 hipError_t launch_compact_table(const Table& t, const int32_t* idx, int64_t n, uint32_t* xo,
                                 int32_t* y, int32_t* z, hipStream_t st);
-// Entailment over a batch: out_idx == nullptr counts (live[k] = propagators
-// not entailed, empty[k] = store holds an empty interval); otherwise writes
-// those propagators' table positions at out_off[k].
-hipError_t launch_batch_ask(const Table& t, const int2* store, int64_t nvars, const Subsets& sub,
-                            int64_t n_props, int64_t n_inst, int64_t* live, int32_t* empty,
-                            const int64_t* out_off, int32_t* out_idx, hipStream_t st);
+// Entailment over a batch (pcx_ask.hip), in chunks of kAskChunk propagators of one
+// instance, `chunks` (ask_chunks of the largest instance) per instance.
+constexpr int kAskChunk = 4096;
+struct AskWork {
+  unsigned long long* bits; // [n_inst * chunks * kAskChunk / 64]: set where not entailed
+  int32_t* count;           // [n_inst * chunks] set bits
+  int64_t* place;           // [n_inst * chunks] set bits of the chunks before
+  int64_t* off;             // [n_inst + 1] set bits of the instances before
+  int32_t* empty;           // [n_inst]: 1 where the store holds an empty interval (zeroed by the caller)
+};
+int64_t ask_chunks(int64_t most_props);
+// everything but the positions
+hipError_t launch_ask_bits(const Table& t, const int2* store, int64_t nvars, const Subsets& sub, int64_t n_props,
+                           int64_t n_inst, int64_t chunks, const AskWork& w, int device, int cus, hipStream_t st);
+// the positions, in the order of the instances, as far as cap
+hipError_t launch_ask_write(const Subsets& sub, int64_t n_inst, int64_t chunks, const AskWork& w, int32_t* out,
+                            int64_t cap, hipStream_t st);
 // Branching: var[k] = split variable of parent instance k (or -1); children
 // 2k / 2k+1 written to child and child_image, and their emptiness (that of
 // their parent) to child_empty when given; one pass over the parents.

@@ -2558,95 +2558,6 @@ hipError_t launch_compact_table(const Table& t, const int32_t* idx, int64_t n, u
   return hipGetLastError();
 }
 
-// ---- entailment over a batch ----------------------------------------------
-// One workgroup per instance (grid-stride over instances).  count: the
-// instance's propagators that are not entailed on its store, and whether the
-// store holds an empty interval.  write: those propagators' table positions,
-// ascending, at out_off[k] (a block scan per 256 propagators keeps the order).
-__device__ __forceinline__ bool inst_prop_entailed(const Table& t, const int2* st,
-                                                   const Subsets& sub, int64_t k, int64_t q,
-                                                   int64_t& p) {
-  p = sub.off ? (int64_t)sub.idx[sub.off[k] + q] : q;
-  const uint32_t xo = t.xo[p];
-  return entailed((int)(xo >> kOpShift), st[xo & kVarMask], st[t.y[p]], st[t.z[p]]);
-}
-
-__global__ __launch_bounds__(kBlock) void k_batch_ask_count(Table t, const int2* __restrict__ store,
-                                                            int64_t nvars, Subsets sub,
-                                                            int64_t n_props, int64_t n_inst,
-                                                            int64_t* live, int32_t* empty) {
-  __shared__ int s_cnt, s_empty;
-  for (int64_t k = blockIdx.x; k < n_inst; k += gridDim.x) {
-    if (threadIdx.x == 0) { s_cnt = 0; s_empty = 0; }
-    __syncthreads();
-    const int2* st = store + k * nvars;
-    const int64_t m = sub.off ? sub.off[k + 1] - sub.off[k] : n_props;
-    int c = 0;
-    for (int64_t q = threadIdx.x; q < m; q += kBlock) {
-      int64_t p;
-      c += !inst_prop_entailed(t, st, sub, k, q, p);
-    }
-    bool e = false;
-    for (int64_t v = threadIdx.x; v < nvars; v += kBlock) e |= st[v].x > st[v].y;
-    c = wave_sum(c);
-    if (lane_id() == 0 && c) atomicAdd(&s_cnt, c);
-    if (__ballot(e) && lane_id() == 0) s_empty = 1;
-    __syncthreads();
-    if (threadIdx.x == 0) { live[k] = s_cnt; empty[k] = s_empty; }
-    __syncthreads();
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void k_batch_ask_write(Table t, const int2* __restrict__ store,
-                                                            int64_t nvars, Subsets sub,
-                                                            int64_t n_props, int64_t n_inst,
-                                                            const int64_t* out_off,
-                                                            int32_t* out_idx) {
-  __shared__ int s_scan[kBlock / kWave];
-  for (int64_t k = blockIdx.x; k < n_inst; k += gridDim.x) {
-    const int2* st = store + k * nvars;
-    const int64_t m = sub.off ? sub.off[k + 1] - sub.off[k] : n_props;
-    int64_t at = out_off[k];
-    for (int64_t q0 = 0; q0 < m; q0 += kBlock) {               // same trip count in every thread
-      const int64_t q = q0 + threadIdx.x;
-      int64_t p = -1;
-      const int keep = q < m && !inst_prop_entailed(t, st, sub, k, q, p);
-      const int lane = lane_id(), wv = threadIdx.x / kWave;
-      int incl = keep;
-#pragma unroll
-      for (int o = 1; o < kWave; o <<= 1) {
-        const int v = __shfl_up(incl, o, kWave);
-        if (lane >= o) incl += v;
-      }
-      if (lane == kWave - 1) s_scan[wv] = incl;
-      __syncthreads();
-      int off = incl - keep, total = 0;
-#pragma unroll
-      for (int i = 0; i < kBlock / kWave; ++i) {
-        if (i < wv) off += s_scan[i];
-        total += s_scan[i];
-      }
-      if (keep) out_idx[at + off] = (int32_t)p;
-      at += total;
-      __syncthreads();                                          // s_scan is rewritten next chunk
-    }
-  }
-}
-
-hipError_t launch_batch_ask(const Table& t, const int2* store, int64_t nvars, const Subsets& sub,
-                            int64_t n_props, int64_t n_inst, int64_t* live, int32_t* empty,
-                            const int64_t* out_off, int32_t* out_idx, hipStream_t stream) {
-  const int64_t grid = n_inst < 65536 ? n_inst : 65536;
-  if (grid <= 0) return hipSuccess;
-  if (!out_idx)
-    k_batch_ask_count<<<(unsigned)grid, kBlock, 0, stream>>>(t, store, nvars, sub, n_props, n_inst,
-                                                            live, empty);
-  else
-    k_batch_ask_write<<<(unsigned)grid, kBlock, 0, stream>>>(t, store, nvars, sub, n_props, n_inst,
-                                                            out_off, out_idx);
-  return hipGetLastError();
-}
-
 // ---- branching: two children per instance ---------------------------------
 // One pass per parent k (a workgroup each): children 2k and 2k+1 (stores
 // and image) are written as copies of the parent while the workgroup finds

@@ -99,25 +99,85 @@ struct NetRoot {
   int64_t nvars = 0;
 };
 
-// out[0] = 1 when the store leaves the told store somewhere.
-__global__ __launch_bounds__(256) void k_root_within(const int2* __restrict__ st, const int2* __restrict__ told,
-                                                     int64_t nvars, int32_t* out) {
+// A tick's admissions and hand-backs are one launch each over lists of items in
+// pinned memory, and the kernels move the stores between the staging buffer (lb,
+// then ub) and the arena themselves: six and three runtime calls per request were
+// most of a tick (48 requests at once: 3.4 ms, of which the device was busy 0.8).
+struct AdmitItem {
+  const int32_t* lb;        // staged bounds
+  const int32_t* ub;
+  int2* store;              // the request's arena block
+  int64_t nvars;
+  const int2* told;         // the network's told store and root fixpoint, or nullptr
+  const int2* root;
+  SlotDesc slot;            // (its marks are zeroed)
+  InstFlags flags;
+  int32_t k;                // slot number
+};
+struct HandBackItem {
+  const int2* store;
+  int32_t* lb;
+  int32_t* ub;
+  int64_t nvars;
+  InstFlags parked;         // the slot's flags from now on
+  int32_t k;
+};
+constexpr int32_t kItems = 1024;        // items of one launch
+constexpr int kItemBlocks = 16;         // workgroups per item
+
+// Stores, mark bitmaps, descriptors and flags of the items; out[k] = 1 when a
+// store leaves its told store somewhere (out zeroed by the caller).
+__global__ __launch_bounds__(256) void k_admit(const AdmitItem* items, SlotDesc* slots, InstFlags* flags, int32_t* out) {
+  const AdmitItem* it = items + blockIdx.y;
+  const int64_t n = it->nvars, i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int32_t *lb = it->lb, *ub = it->ub;
+  int2* const st = it->store;
+  const int2* const told = it->told;
   bool outside = false;
-  for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < nvars; v += (int64_t)gridDim.x * 256) {
-    const int2 a = st[v], t = told[v];
-    outside |= a.x < t.x || a.y > t.y;
+  for (int64_t v = i0; v < n; v += kItemBlocks * 256) {
+    const int2 a = make_int2(lb[v], ub[v]);
+    st[v] = a;
+    if (told) {
+      const int2 t = told[v];
+      outside |= a.x < t.x || a.y > t.y;
+    }
   }
-  if (__ballot(outside) && (threadIdx.x & 63) == 0) *out = 1;
+  uint32_t* const marks = it->slot.marks;
+  const int64_t mw = marks ? 2 * it->slot.words + 3 * it->slot.swords : 0;
+  for (int64_t w = i0; w < mw; w += kItemBlocks * 256) marks[w] = 0;
+  if (__ballot(outside) && (threadIdx.x & 63) == 0) out[it->k] = 1;
+  if (i0 == 0) {
+    slots[it->k] = it->slot;
+    flags[it->k] = it->flags;
+  }
 }
 
-// Unless out[0] is set: the store meets the root fixpoint.
-__global__ __launch_bounds__(256) void k_root_meet(int2* __restrict__ st, const int2* __restrict__ root,
-                                                   int64_t nvars, const int32_t* out) {
-  if (*out) return;
-  for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < nvars; v += (int64_t)gridDim.x * 256) {
+// The items with a root whose store lies inside the told one: the store meets the
+// root fixpoint.
+__global__ __launch_bounds__(256) void k_admit_meet(const AdmitItem* items, const int32_t* out) {
+  const AdmitItem* it = items + blockIdx.y;
+  const int2* const root = it->root;
+  if (!root || out[it->k]) return;
+  int2* const st = it->store;
+  const int64_t n = it->nvars;
+  for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += kItemBlocks * 256) {
     const int2 a = st[v], r = root[v];
     st[v] = make_int2(max(a.x, r.x), min(a.y, r.y));
   }
+}
+
+// Finished stores into the staging buffer, and their slots parked.
+__global__ __launch_bounds__(256) void k_hand_back(const HandBackItem* items, InstFlags* flags) {
+  const HandBackItem* it = items + blockIdx.y;
+  const int64_t n = it->nvars, i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int2* const st = it->store;
+  int32_t *lb = it->lb, *ub = it->ub;
+  for (int64_t v = i0; v < n; v += kItemBlocks * 256) {
+    const int2 a = st[v];
+    lb[v] = a.x;
+    ub[v] = a.y;
+  }
+  if (i0 == 0) flags[it->k] = it->parked;
 }
 
 // Side lanes: concurrent burst launches, each on a stream of its own (with
@@ -148,7 +208,9 @@ struct pcx_server {
   std::vector<Slot> slots;
   SlotDesc* h_slots = nullptr;        // pinned mirrors
   InstFlags* h_flags = nullptr;
-  int2* h_stage = nullptr;            // pinned staging ring for store uploads
+  int2* h_stage = nullptr;            // pinned staging buffer of stores (a store's lb, then its ub)
+  AdmitItem* h_admit = nullptr;       // pinned lists of one launch's items
+  HandBackItem* h_back = nullptr;
   int64_t stage_words = 0;
   std::deque<Request> pending;
   std::vector<pcx_served> done;
@@ -211,14 +273,27 @@ void finish(pcx_server* s, const Request& rq, const pcx_result& r) {
   ++s->stats.completed;
 }
 
-// Move queued requests into free slots while the arena and staging ring
+// Launch the first n admissions of h_admit.
+pcx_status admit_items(pcx_server* s, int32_t n) {
+  if (n == 0) return PCX_OK;
+  PCX_HIP(hipMemsetAsync(s->d_root_out, 0, s->n_slots * sizeof(int32_t), s->stream));
+  k_admit<<<dim3(kItemBlocks, n), 256, 0, s->stream>>>(s->h_admit, s->d_slots, s->d_flags, s->d_root_out);
+  k_admit_meet<<<dim3(kItemBlocks, n), 256, 0, s->stream>>>(s->h_admit, s->d_root_out);
+  PCX_HIP(hipGetLastError());
+  return PCX_OK;
+}
+
+// Move queued requests into free slots while the arena and staging buffer
 // have room.  Stores with an empty domain finish at once (failed, 0 sweeps).
+// The staging buffer and h_admit are free on entry (the last tick waited for its
+// launches), and the tick waits for these.
 pcx_status admit(pcx_server* s) {
   int64_t staged = 0;
+  int32_t items = 0;
   while (!s->pending.empty()) {
     Request& rq = s->pending.front();
     bool empty = false;
-    for (int64_t v = 0; v < rq.nvars && !empty; ++v) empty = rq.lb[v] > rq.ub[v];
+    for (int64_t v = 0; v < rq.nvars; ++v) empty |= rq.lb[v] > rq.ub[v];
     if (empty) {
       pcx_result r{};
       r.failed = 1;
@@ -234,18 +309,20 @@ pcx_status admit(pcx_server* s) {
     const Footprint fp = footprint(s, rq);
     const int64_t off = s->arena.alloc(fp.units);
     if (off < 0) { ++s->stats.waits_arena; break; }   // no HBM room: wait for a slot to drain
-    int2* stage = s->h_stage + staged;
-    for (int64_t v = 0; v < rq.nvars; ++v) stage[v] = make_int2(rq.lb[v], rq.ub[v]);
-    PCX_HIP(hipMemcpyAsync(s->d_arena + off, stage, rq.nvars * sizeof(int2), hipMemcpyHostToDevice, s->stream));
+    int32_t* stage = reinterpret_cast<int32_t*>(s->h_stage + staged);
+    std::memcpy(stage, rq.lb, rq.nvars * sizeof(int32_t));
+    std::memcpy(stage + rq.nvars, rq.ub, rq.nvars * sizeof(int32_t));
     staged += rq.nvars;
+    AdmitItem it{};
+    it.lb = stage;
+    it.ub = stage + rq.nvars;
+    it.store = s->d_arena + off;
+    it.nvars = rq.nvars;
+    it.k = k;
     if (rq.net < (int32_t)s->roots.size() && s->roots[rq.net].root && s->roots[rq.net].nvars == rq.nvars) {
       // inside the told store: start from the meet with the root fixpoint
-      const NetRoot& nr = s->roots[rq.net];
-      const unsigned g = (unsigned)std::min<int64_t>((rq.nvars + 255) / 256, 2048);
-      PCX_HIP(hipMemsetAsync(s->d_root_out + k, 0, sizeof(int32_t), s->stream));
-      k_root_within<<<g, 256, 0, s->stream>>>(s->d_arena + off, nr.told, rq.nvars, s->d_root_out + k);
-      k_root_meet<<<g, 256, 0, s->stream>>>(s->d_arena + off, nr.root, rq.nvars, s->d_root_out + k);
-      PCX_HIP(hipGetLastError());
+      it.told = s->roots[rq.net].told;
+      it.root = s->roots[rq.net].root;
     }
     pcx_engine* e = s->nets[rq.net];
     const int32_t S = s->next_sweep;
@@ -262,7 +339,6 @@ pcx_status admit(pcx_server* s) {
       sd.marks = reinterpret_cast<uint32_t*>(s->d_arena + off + rq.nvars);
       sd.words = fp.words;
       sd.swords = fp.swords;
-      PCX_HIP(hipMemsetAsync(sd.marks, 0, (2 * fp.words + 3 * fp.swords) * sizeof(uint32_t), s->stream));
     }
     s->h_slots[k] = sd;
     InstFlags f{};
@@ -273,8 +349,9 @@ pcx_status admit(pcx_server* s) {
     f.settled_at = -1;
     f.all_marked[0] = f.all_marked[1] = -1;
     s->h_flags[k] = f;
-    pcx_status st = upload_slot_meta(s, k);
-    if (st != PCX_OK) return st;
+    it.slot = sd;
+    it.flags = f;
+    s->h_admit[items++] = it;
     Slot& sl = s->slots[k];
     sl.busy = true;
     sl.req = rq;
@@ -288,8 +365,14 @@ pcx_status admit(pcx_server* s) {
     ++s->stats.admitted;
     s->stats.arena_peak_bytes = std::max(s->stats.arena_peak_bytes,
                                          (int64_t)((off + fp.units) * sizeof(int2)));
+    if (items == kItems) {                     // the list is full: launch it and wait to reuse it
+      pcx_status st = admit_items(s, items);
+      if (st != PCX_OK) return st;
+      PCX_HIP(hipStreamSynchronize(s->stream));
+      items = 0;
+    }
   }
-  return PCX_OK;
+  return admit_items(s, items);
 }
 
 // A slot's result from its flags: slot-batch sweeps up to the failing /
@@ -319,40 +402,46 @@ pcx_result result_of(const pcx_server* s, int32_t k, const InstFlags& f) {
 // Hand back finished slots (flags in fl): their stores are copied back
 // together (one synchronization), then their slot and arena block are freed.
 pcx_status complete(pcx_server* s, const std::vector<int32_t>& ks, const InstFlags* fl) {
-  if (ks.empty()) return PCX_OK;
-  std::vector<int64_t> at;
-  int64_t staged = 0;
-  for (int32_t k : ks) {
-    const Slot& sl = s->slots[k];
-    PCX_HIP(hipMemcpyAsync(s->h_stage + staged, s->d_arena + sl.off, sl.req.nvars * sizeof(int2),
-                           hipMemcpyDeviceToHost, s->stream));
-    at.push_back(staged);
-    staged += sl.req.nvars;
-  }
-  PCX_HIP(hipStreamSynchronize(s->stream));
-  for (size_t i = 0; i < ks.size(); ++i) {
-    const int32_t k = ks[i];
-    Slot& sl = s->slots[k];
-    pcx_result r = result_of(s, k, fl[k]);
-    const int2* stage = s->h_stage + at[i];
-    bool moved = false;                          // the fixpoint differs from the request's store
-    for (int64_t v = 0; v < sl.req.nvars; ++v) {
-      moved |= sl.req.lb[v] != stage[v].x || sl.req.ub[v] != stage[v].y;
-      sl.req.lb[v] = stage[v].x;
-      sl.req.ub[v] = stage[v].y;
+  for (size_t i0 = 0; i0 < ks.size(); i0 += kItems) {
+    const int32_t n = (int32_t)std::min<size_t>(kItems, ks.size() - i0);
+    int64_t staged = 0;
+    for (int32_t i = 0; i < n; ++i) {
+      const int32_t k = ks[i0 + i];
+      const Slot& sl = s->slots[k];
+      HandBackItem it{};
+      it.store = s->d_arena + sl.off;
+      it.lb = reinterpret_cast<int32_t*>(s->h_stage + staged);
+      it.ub = it.lb + sl.req.nvars;
+      it.nvars = sl.req.nvars;
+      it.k = k;
+      it.parked = fl[k];                       // never scheduled until re-admitted
+      it.parked.failed_at = kFreeFailed;
+      it.parked.done_at = 0;
+      s->h_back[i] = it;
+      staged += sl.req.nvars;
     }
-    // (a request started from its meet with a root fixpoint may change
-    // nothing on the device and still differ from its own store)
-    if (!r.failed) r.has_changed = moved;
-    finish(s, sl.req, r);
-    s->arena.release(sl.off, sl.units);
-    sl.busy = false;
-    sl.side = false;
-    // park the slot: never scheduled until re-admitted
-    s->h_flags[k].failed_at = kFreeFailed;
-    s->h_flags[k].done_at = 0;
-    pcx_status st = upload_slot_meta(s, k);
-    if (st != PCX_OK) return st;
+    k_hand_back<<<dim3(kItemBlocks, n), 256, 0, s->stream>>>(s->h_back, s->d_flags);
+    PCX_HIP(hipGetLastError());
+    PCX_HIP(hipStreamSynchronize(s->stream));
+    for (int32_t i = 0; i < n; ++i) {
+      const int32_t k = ks[i0 + i];
+      Slot& sl = s->slots[k];
+      pcx_result r = result_of(s, k, fl[k]);
+      const HandBackItem& it = s->h_back[i];
+      const int64_t nv = sl.req.nvars;
+      int32_t moved = 0;                       // the fixpoint differs from the request's store
+      for (int64_t v = 0; v < nv; ++v) moved |= (sl.req.lb[v] ^ it.lb[v]) | (sl.req.ub[v] ^ it.ub[v]);
+      std::memcpy(sl.req.lb, it.lb, nv * sizeof(int32_t));
+      std::memcpy(sl.req.ub, it.ub, nv * sizeof(int32_t));
+      // (a request started from its meet with a root fixpoint may change
+      // nothing on the device and still differ from its own store)
+      if (!r.failed) r.has_changed = moved != 0;
+      finish(s, sl.req, r);
+      s->arena.release(sl.off, sl.units);
+      sl.busy = false;
+      sl.side = false;
+      s->h_flags[k] = it.parked;
+    }
   }
   return PCX_OK;
 }
@@ -607,7 +696,7 @@ void pcx_server_destroy(pcx_server* s) {
   for (void* p : {(void*)s->d_slots, (void*)s->d_flags, (void*)s->d_act, (void*)s->d_item_base,
                   (void*)s->d_ctl, (void*)s->d_tight, (void*)s->d_arena})
     if (p) (void)hipFree(p);
-  for (void* p : {(void*)s->h_slots, (void*)s->h_flags, (void*)s->h_stage})
+  for (void* p : {(void*)s->h_slots, (void*)s->h_flags, (void*)s->h_stage, (void*)s->h_admit, (void*)s->h_back})
     if (p) (void)hipHostFree(p);
   for (SideLane& ln : s->lanes) {
     if (ln.h_flags) (void)hipHostFree(ln.h_flags);
@@ -658,6 +747,7 @@ pcx_status pcx_server_create(const pcx_server_config* cfg, pcx_server** out) {
   }
   chk(hipMalloc(&s->d_slots, c.max_slots * sizeof(SlotDesc)));
   chk(hipMalloc(&s->d_flags, c.max_slots * sizeof(InstFlags)));
+  chk(hipMalloc(&s->d_root_out, c.max_slots * sizeof(int32_t)));
   chk(hipMalloc(&s->d_act, c.max_slots * sizeof(int32_t)));
   chk(hipMalloc(&s->d_item_base, (c.max_slots + 1) * sizeof(int64_t)));
   chk(hipMalloc(&s->d_ctl, kCtlWords * sizeof(int32_t)));
@@ -666,6 +756,8 @@ pcx_status pcx_server_create(const pcx_server_config* cfg, pcx_server** out) {
   chk(hipHostMalloc(&s->h_slots, c.max_slots * sizeof(SlotDesc), hipHostMallocDefault));
   chk(hipHostMalloc(&s->h_flags, c.max_slots * sizeof(InstFlags), hipHostMallocDefault));
   chk(hipHostMalloc(&s->h_stage, s->stage_words * sizeof(int2), hipHostMallocDefault));
+  chk(hipHostMalloc(&s->h_admit, kItems * sizeof(AdmitItem), hipHostMallocDefault));
+  chk(hipHostMalloc(&s->h_back, kItems * sizeof(HandBackItem), hipHostMallocDefault));
   if (he != hipSuccess) {
     pcx_server_destroy(s);
     return fail_with(he == hipErrorOutOfMemory ? PCX_ENOMEM : PCX_EDEVICE,
@@ -729,7 +821,6 @@ pcx_status pcx_server_set_root(pcx_server* s, int32_t net, const int32_t* lb, co
     told[v] = make_int2(lb[v], ub[v]);
     root[v] = make_int2(rl[v], ru[v]);
   }
-  if (!s->d_root_out) PCX_HIP(hipMalloc(&s->d_root_out, s->n_slots * sizeof(int32_t)));
   if ((int32_t)s->roots.size() <= net) s->roots.resize(net + 1);
   NetRoot& nr = s->roots[net];
   PCX_HIP(hipStreamSynchronize(s->stream));        // no admission still reads the old root

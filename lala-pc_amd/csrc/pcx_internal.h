@@ -91,6 +91,10 @@ struct pcx_batch {
                                       // then [n_inst * kSeedCap] the drain's seeds
   int32_t* d_trail_n = nullptr;       // [2 * n_inst]: the two lists' counts
   bool trail_valid = false;           // the stores are the image but for the trail's variables
+  int2* d_undo = nullptr;             // [n_inst * kTrailCap] the values of the trail's variables before
+  bool image_absent = false;          // nothing holds the image but the stores themselves, or (after
+                                      // a drained run) the stores and the undo log: a branching that
+                                      // seeded a drain
   uint8_t* d_ask = nullptr;           // arrays of the last ask, kept for the next
   int64_t ask_bytes = 0;
   int32_t device = 0;                 // the engine's device (destroy reads it, not the engine)

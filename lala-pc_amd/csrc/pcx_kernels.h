@@ -271,7 +271,13 @@ hipError_t launch_seed_from_base(const EventSet& ev, const DiffSink& diffs, int6
 // restore rewrites only those.
 hipError_t launch_drain_marks(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
                               int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
-                              const InstLists& trail, int dom, int grid, hipStream_t st);
+                              const InstLists& trail, int2* undo, int2* image, int dom, int grid, hipStream_t st);
+// A drain with undo ([n_inst * trail.cap] values) also lists, beside each variable
+// of the trail, the value it was tightened from, and writes an instance's row of
+// image before its trail overflows.  launch_undo: dst (the stores, or the image)
+// as the stores were before that drain.
+hipError_t launch_undo(const InstLists& trail, const int2* undo, const int2* store, const int2* image, int2* dst,
+                       int64_t nvars, int64_t n_inst, int dom, hipStream_t st);
 // The stores back to their image after a drained run with a trail: each
 // instance's listed variables (its whole row when the list is incomplete)
 // from the image, which is either d_image or the base store plus the listed
@@ -378,7 +384,7 @@ hipError_t launch_ask_bits(const Table& t, const int2* store, int64_t nvars, con
 hipError_t launch_ask_write(const Subsets& sub, int64_t n_inst, int64_t chunks, const AskWork& w, int32_t* out,
                             int64_t cap, hipStream_t st);
 // Branching: var[k] = split variable of parent instance k (or -1); children
-// 2k / 2k+1 written to child and child_image, and their emptiness (that of
+// 2k / 2k+1 written to child and (when given) child_image, and their emptiness (that of
 // their parent) to child_empty when given; one pass over the parents.
 hipError_t launch_branch(const int2* parent, int64_t nvars, int64_t n_inst, int32_t* var, int2* child,
                          int2* child_image, uint8_t* child_empty, int dom, hipStream_t st);

@@ -2559,8 +2559,8 @@ hipError_t launch_compact_table(const Table& t, const int32_t* idx, int64_t n, u
 }
 
 // ---- branching: two children per instance ---------------------------------
-// One pass per parent k (a workgroup each): children 2k and 2k+1 (stores
-// and image) are written as copies of the parent while the workgroup finds
+// One pass per parent k (a workgroup each): children 2k and 2k+1 (stores, and
+// image when given) are written as copies of the parent while the workgroup finds
 // var[k], the first variable (input order) that is not fixed (-1 when the
 // store is empty or every variable is fixed), and whether the store is
 // empty; then that variable is split in both children: intervals
@@ -2591,8 +2591,8 @@ __global__ __launch_bounds__(kBlock) void k_branch(const int2* __restrict__ pare
     const int2* p = parent + k * nvars;
     int2* c0 = child + 2 * k * nvars;
     int2* c1 = c0 + nvars;
-    int2* i0 = child_image + 2 * k * nvars;
-    int2* i1 = i0 + nvars;
+    int2* i0 = child_image ? child_image + 2 * k * nvars : nullptr;
+    int2* i1 = child_image ? i0 + nvars : nullptr;
     int32_t first = 0x7fffffff;
     bool empty = false;
     if constexpr (V2) {
@@ -2603,8 +2603,10 @@ __global__ __launch_bounds__(kBlock) void k_branch(const int2* __restrict__ pare
         const int4 b = p4[h];
         c04[h] = b;
         c14[h] = b;
-        i04[h] = b;
-        i14[h] = b;
+        if (child_image) {
+          i04[h] = b;
+          i14[h] = b;
+        }
         branch_scan<BITS>(make_int2(b.x, b.y), (int32_t)(2 * h), first, empty);
         branch_scan<BITS>(make_int2(b.z, b.w), (int32_t)(2 * h + 1), first, empty);
       }
@@ -2613,8 +2615,10 @@ __global__ __launch_bounds__(kBlock) void k_branch(const int2* __restrict__ pare
         const int2 b = p[v];
         c0[v] = b;
         c1[v] = b;
-        i0[v] = b;
-        i1[v] = b;
+        if (child_image) {
+          i0[v] = b;
+          i1[v] = b;
+        }
         branch_scan<BITS>(b, (int32_t)v, first, empty);
       }
     }
@@ -2640,8 +2644,10 @@ __global__ __launch_bounds__(kBlock) void k_branch(const int2* __restrict__ pare
         }
         c0[sv] = left;
         c1[sv] = right;
-        i0[sv] = left;
-        i1[sv] = right;
+        if (child_image) {
+          i0[sv] = left;
+          i1[sv] = right;
+        }
       }
     }
     __syncthreads();                             // s_first / s_empty read before the next parent
@@ -2995,6 +3001,55 @@ hipError_t launch_restore_trail(const InstLists& tr, const DiffSink& ds, const i
   return hipGetLastError();
 }
 
+// Undo logs (InstLists of variables, and beside each entry the value the
+// variable held when the drain tightened it): a domain only shrinks, and the first
+// thread to tighten a bound (or to remove a value) read it as it was at the start,
+// so the loosest of a variable's entries is its value at the start.
+template <bool BITS>
+__device__ __forceinline__ void undo_value(u64* row, int32_t v, u64 old) {
+  constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
+  if constexpr (BITS) {
+    __hip_atomic_fetch_or(&row[v], old, __ATOMIC_RELAXED, WG);
+  } else {
+    int2* r = reinterpret_cast<int2*>(row) + v;
+    __hip_atomic_fetch_min(&r->x, as_itv(old).x, __ATOMIC_RELAXED, WG);
+    __hip_atomic_fetch_max(&r->y, as_itv(old).y, __ATOMIC_RELAXED, WG);
+  }
+}
+
+// dst's rows as the stores were before the drain.  dst == store: the stores
+// themselves are restored; otherwise the rows are copied first.  The row of an
+// instance whose log is incomplete lies in image (and is left there when dst is
+// the image).
+template <bool BITS>
+__global__ __launch_bounds__(kBlock) void k_undo(InstLists tr, const u64* __restrict__ undo, const u64* store,
+                                                 const u64* image, u64* dst, int64_t nvars, int64_t n_inst) {
+  for (int64_t k = blockIdx.x; k < n_inst; k += gridDim.x) {
+    const int32_t n = tr.n[k];
+    u64* row = dst + k * nvars;
+    const u64* from = n <= tr.cap ? store : image;
+    if (from != dst)
+      for (int64_t v = threadIdx.x; v < nvars; v += kBlock) row[v] = from[k * nvars + v];
+    if (n > tr.cap) continue;                          // the same for every thread
+    __syncthreads();
+    const int32_t* list = tr.list + k * tr.cap;
+    for (int i = threadIdx.x; i < n; i += kBlock) undo_value<BITS>(row, list[i], undo[k * tr.cap + i]);
+  }
+}
+
+hipError_t launch_undo(const InstLists& tr, const int2* undo, const int2* store, const int2* image, int2* dst,
+                       int64_t nvars, int64_t n_inst, int dom, hipStream_t stream) {
+  if (nvars <= 0 || n_inst <= 0) return hipSuccess;
+  if (!tr.list || !undo) return hipErrorInvalidValue;
+  const unsigned grid = (unsigned)(n_inst < 65536 ? n_inst : 65536);
+  const u64 *u = reinterpret_cast<const u64*>(undo), *st = reinterpret_cast<const u64*>(store);
+  const u64* im = reinterpret_cast<const u64*>(image);
+  u64* d = reinterpret_cast<u64*>(dst);
+  if (dom == kBits) k_undo<true><<<grid, kBlock, 0, stream>>>(tr, u, st, im, d, nvars, n_inst);
+  else k_undo<false><<<grid, kBlock, 0, stream>>>(tr, u, st, im, d, nvars, n_inst);
+  return hipGetLastError();
+}
+
 // The base value at every listed difference's position.
 __global__ __launch_bounds__(kBlock) void k_unscatter_diffs(DiffSink ds, u64* __restrict__ store, int64_t nvars) {
   const u64* base = reinterpret_cast<const u64*>(ds.base);
@@ -3263,12 +3318,19 @@ __device__ __forceinline__ void drain_scan(uint32_t* row, int64_t words, bool fi
   }
 }
 
-template <int D, int B>
+// UNDO: the trail keeps each variable's value beside it (undo), and an instance
+// whose trail the next round might overfill (three variables a propagator) gets
+// its row of the image first: the row as it is now, with the trail's values put
+// back.  (The children of a branching: the few values logged replace 0.82 GB of image
+// written per branching of 1,024 nodes of 50,000 variables; the drain itself takes
+// what it took.)
+template <int D, int B, bool UNDO>
 __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ store, int64_t nvars,
                                                    InstFlags* flags, EventSet ev, int32_t* next_inst,
                                                    unsigned long long* tight, InstLists seeds,
-                                                   InstLists trail) {
+                                                   InstLists trail, u64* undo, u64* image) {
   constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
+  __shared__ u64 s_old[UNDO ? kDrainVars : 1];
   __shared__ int32_t s_list[2][kWorkCap];
   __shared__ int32_t s_hash[kDrainHash];
   __shared__ int32_t s_tv[kDrainVars];
@@ -3291,10 +3353,13 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
     }
     int32_t* tlist = trail.list ? trail.list + k * trail.cap : nullptr;
     // a tightened variable on the trail (past the cap only counted)
-    auto on_trail = [&](int32_t v) {
+    auto on_trail = [&](int32_t v, u64 old) {
       if (!tlist) return;
       const int at = atomicAdd(&s_tn, 1);
-      if (at < trail.cap) tlist[at] = v;
+      if (at < trail.cap) {
+        tlist[at] = v;
+        if (UNDO) undo[k * trail.cap + at] = old;
+      }
     };
     const uint32_t* mrow = ev.member ? ev.member + k * ev.words : nullptr;
     int2* st = store + k * nvars;
@@ -3323,6 +3388,15 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
       }
       const int n = min(s_n[cur], kWorkCap);
       if (n == 0) break;                               // nothing marked: the fixpoint
+      if (UNDO && s_tn <= trail.cap && s_tn + 3 * n > trail.cap) {   // the same in every thread
+        u64* irow = image + k * nvars;
+        for (int64_t v = tid; v < nvars; v += B) irow[v] = load_word<WG>(st + v);
+        __syncthreads();
+        const int tn = s_tn;
+        for (int i = tid; i < tn; i += B) undo_value<D == kBits>(irow, tlist[i], undo[k * trail.cap + i]);
+        __syncthreads();                               // every thread has read s_tn and the trail
+        if (tid == 0) s_tn = trail.cap + 1;            // restored whole, from the image
+      }
       if (tid == 0) { s_n[nx] = 0; s_over[nx] = s_over[cur]; s_chg = 0; s_fail = 0; s_ntv = 0; }
       for (int i = tid; i < kDrainHash; i += B) s_hash[i] = -1;
       __syncthreads();
@@ -3364,15 +3438,17 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
         chg |= c;
         fail |= fl;
         const int32_t vs[3] = {x, y, z};
+        const u64 ws[3] = {wx, wy, wz};
         const bool ts[3] = {tx, ty, tz};
         for (int j = 0; j < 3; ++j) {
           if (!ts[j]) continue;
           const int at = atomicAdd(&s_ntv, 1);
           if (at < kDrainVars) {
             s_tv[at] = vs[j];
+            if (UNDO) s_old[at] = ws[j];
           } else {
             drain_mark(row, mrow, ev, vs[j], s_hash, s_list[nx], &s_n[nx], &s_over[nx]);
-            on_trail(vs[j]);
+            on_trail(vs[j], ws[j]);
           }
         }
       }
@@ -3381,7 +3457,7 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
       const int ntv = min(s_ntv, kDrainVars);
       for (int i = tid; i < ntv; i += B) {
         drain_mark(row, mrow, ev, s_tv[i], s_hash, s_list[nx], &s_n[nx], &s_over[nx]);
-        on_trail(s_tv[i]);
+        on_trail(s_tv[i], UNDO ? s_old[i] : 0);
       }
       if (__ballot(chg) && lane_id() == 0) s_chg = 1;
       if (__ballot(fail) && lane_id() == 0) s_fail = 1;
@@ -3406,22 +3482,38 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
     atomicAdd(&tight[blockIdx.x & (kTightSlots - 1)], (unsigned long long)sum);
 }
 
-hipError_t launch_drain_marks(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
-                              int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
-                              const InstLists& trail, int dom, int grid, hipStream_t stream) {
-  if (ev.n_inst <= 0 || !ev.dirty) return hipSuccess;
+namespace {
+template <bool UNDO>
+hipError_t launch_drain_u(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
+                          int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
+                          const InstLists& trail, u64* undo, u64* image, int dom, int grid, hipStream_t stream) {
   // Workgroups of two waves: at 4,096 interval instances of 50,000 variables
   // 0.228 ms against 0.236 with one wave and 0.255 with four (the replayed
   // step 0.33 ms against 0.35-0.36); at 1,024 bitset instances of 200,000
   // words 98 us against 105 with one wave.
   constexpr int kDrainB = 2 * kWave;
+#define PCX_DRAIN(D) \
+  k_drain_marks<D, kDrainB, UNDO><<<grid, kDrainB, 0, stream>>>(t, store, nvars, flags, ev, next_inst, tight, seeds, \
+                                                                trail, undo, image)
   switch (dom) {
-    case kItv: k_drain_marks<kItv, kDrainB><<<grid, kDrainB, 0, stream>>>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail); break;
-    case kItvDiv: k_drain_marks<kItvDiv, kDrainB><<<grid, kDrainB, 0, stream>>>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail); break;
-    case kBits: k_drain_marks<kBits, kDrainB><<<grid, kDrainB, 0, stream>>>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail); break;
+    case kItv: PCX_DRAIN(kItv); break;
+    case kItvDiv: PCX_DRAIN(kItvDiv); break;
+    case kBits: PCX_DRAIN(kBits); break;
     default: return hipErrorInvalidValue;
   }
+#undef PCX_DRAIN
   return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_drain_marks(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
+                              int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
+                              const InstLists& trail, int2* undo, int2* image, int dom, int grid, hipStream_t stream) {
+  if (ev.n_inst <= 0 || !ev.dirty) return hipSuccess;
+  if (undo && (!image || !trail.list)) return hipErrorInvalidValue;
+  u64 *u = reinterpret_cast<u64*>(undo), *im = reinterpret_cast<u64*>(image);
+  return undo ? launch_drain_u<true>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail, u, im, dom, grid, stream)
+              : launch_drain_u<false>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail, u, im, dom, grid, stream);
 }
 
 hipError_t launch_seed_from_base(const EventSet& ev, const DiffSink& diffs, int64_t n_diffs,

@@ -612,14 +612,15 @@ pcx_status prepare_run(pcx_batch* b, int32_t mode, SeedPlan* plan, bool* local) 
     s = write_absent_image(b);
     if (s != PCX_OK) return s;
   }
-  PCX_HIP(hipMemsetAsync(b->d_tight, 0, 2 * kTightSlots * sizeof(unsigned long long), e->stream));
+  int32_t* seed_n = b->d_trail_n ? b->d_trail_n + b->n_inst : nullptr;
   const WorkList wl = worklist_of(b->d_act, b->d_item_base, b->d_ctl);
   // A store already empty is failed before any sweep; when the stores are the
   // image, its emptiness was found at load time.
   if (b->store_is_image) {
-    PCX_HIP(launch_init_flags(b->d_flags, (int32_t)b->n_inst, wl, e->stream, b->d_image_empty));
+    PCX_HIP(launch_init_flags(b->d_flags, (int32_t)b->n_inst, wl, e->stream, b->d_image_empty, b->d_tight,
+                              seed_n));
   } else {
-    PCX_HIP(launch_init_flags(b->d_flags, (int32_t)b->n_inst, wl, e->stream));
+    PCX_HIP(launch_init_flags(b->d_flags, (int32_t)b->n_inst, wl, e->stream, nullptr, b->d_tight, seed_n));
     PCX_HIP(launch_store_check_empty(b->d_store, b->nvars, (int32_t)b->n_inst, b->d_flags, dom_of(e),
                                      e->stream));
   }
@@ -926,11 +927,12 @@ pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, 
   // nor queues.
   InstLists seeds{nullptr, nullptr, 0};
   if (drain) {
+    const bool counts = b->d_trail_n != nullptr;       // zeroed with the flags
     const pcx_status ls = ensure_trail(b);
     if (ls != PCX_OK) return ls;
     if (base_seeded) {                   // a branching's seeds are bits in the rows
       seeds = InstLists{b->d_trail + b->n_inst * kTrailCap, b->d_trail_n + b->n_inst, kSeedCap};
-      PCX_HIP(hipMemsetAsync(seeds.n, 0, b->n_inst * sizeof(int32_t), e->stream));
+      if (!counts) PCX_HIP(hipMemsetAsync(seeds.n, 0, b->n_inst * sizeof(int32_t), e->stream));
     }
   }
   if (base_seeded) {
@@ -940,7 +942,6 @@ pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, 
                                   b->d_unsat, n_unsat, seeds, e->stream));
   }
   if (drain) {
-    PCX_HIP(hipMemsetAsync(b->d_ctl + 3, 0, sizeof(int32_t), e->stream));
     const int dgrid = (int)std::min<int64_t>(b->n_inst, (int64_t)pcx_internal::device_cus(e->cfg.device) * 24);
     pcx_status ts = tm.begin(e->stream);
     if (ts != PCX_OK) return ts;
@@ -952,12 +953,10 @@ pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, 
     std::vector<InstFlags> flags;
     ts = collect(b, flags, results, stats, tm);        // one synchronization for the drain and the flags
     // the drain took and cleared every mark (rows of failed instances too;
-    // a branching's seeds also set summary bits, cleared here), and it started
+    // a branching's seeds set summary bits, which it cleared too), and it started
     // from the image: the stores differ from it only in the trail's variables
     if (ts == PCX_OK) {
       b->trail_valid = b->run_from_image;
-      if (!base_seeded)
-        PCX_HIP(hipMemsetAsync(b->d_summary, 0, 2 * b->n_inst * summary_words(b) * sizeof(uint32_t), e->stream));
       b->marks_clean = true;
     }
     return ts;
@@ -1429,9 +1428,9 @@ pcx_status ensure_diff_list(pcx_batch* b) {
 }
 
 // Where this load lists the differences from the base store (batches of
-// several instances with seeding on), after clearing the counts; an empty
-// sink otherwise.
-pcx_status diff_sink(pcx_batch* b, DiffSink* ds) {
+// several instances with seeding on), after clearing the counts (clear); an
+// empty sink otherwise.
+pcx_status diff_sink(pcx_batch* b, DiffSink* ds, bool clear = true) {
   *ds = DiffSink{nullptr, nullptr, 0, nullptr, nullptr};
   b->diffs_listed = false;
   b->probe_valid = false;
@@ -1440,7 +1439,7 @@ pcx_status diff_sink(pcx_batch* b, DiffSink* ds) {
     return PCX_OK;
   pcx_status st = ensure_diff_list(b);
   if (st != PCX_OK) return st;
-  PCX_HIP(hipMemsetAsync(b->d_seedctl, 0, kSeedCtlWords * sizeof(int32_t), e->stream));
+  if (clear) PCX_HIP(hipMemsetAsync(b->d_seedctl, 0, kSeedCtlWords * sizeof(int32_t), e->stream));
   *ds = DiffSink{b->d_diff, b->d_seedctl, b->diff_cap, b->d_base, b->d_diff_val};
   return PCX_OK;
 }
@@ -1477,8 +1476,7 @@ pcx_status probe_loaded(pcx_batch* b, bool* complete) {
   const bool probe = b->table_n > 0 && (int64_t)e->op.size() == b->table_n;
   if (probe) {
     if (!b->d_unsat) PCX_HIP(hipMalloc(&b->d_unsat, b->table_n * sizeof(int32_t)));
-    int32_t* unsat_n = b->d_seedctl + kDiffLists;      // the probe appends from zero
-    PCX_HIP(hipMemsetAsync(unsat_n, 0, sizeof(int32_t), e->stream));
+    int32_t* unsat_n = b->d_seedctl + kDiffLists;      // cleared with the differences' counts
     PCX_HIP(launch_base_probe(table_of(e), b->d_base, b->d_unsat, unsat_n, dom_of(e), e->stream));
   }
   int32_t ctl[kDiffLists + 1];
@@ -1556,13 +1554,13 @@ pcx_status pcx_batch_load_device(pcx_batch* b, const int32_t* d_lb, const int32_
                                   b->d_store, b->nvars, b->n_inst, e->stream));
     std::swap(b->d_base, b->d_base_alt);   // d_base_alt: what every row now holds
   }
-  PCX_HIP(hipMemsetAsync(b->d_image_empty, 0, b->n_inst, e->stream));
   DiffSink ds;
-  pcx_status dst = diff_sink(b, &ds);
+  pcx_status dst = diff_sink(b, &ds, !b->shared_loads);
   if (dst != PCX_OK) return dst;
   const int gi = lockstep_of(b);
   const bool rows = ds.list && b->shared_loads;
-  if (rows) PCX_HIP(launch_make_base_rows(d_lb, d_ub, b->nvars, b->n_inst, ds, e->stream));
+  if (rows) PCX_HIP(launch_make_base_rows(d_lb, d_ub, b->nvars, b->n_inst, ds, b->d_image_empty, e->stream));
+  else PCX_HIP(hipMemsetAsync(b->d_image_empty, 0, b->n_inst, e->stream));
   // config.timing: HIP events around the load's pass over the stores
   hipEvent_t t0 = nullptr, t1 = nullptr;
   bool t1_recorded = false;

@@ -209,7 +209,7 @@ hipError_t launch_interleave(const int2* store, int2* shadow, int64_t nvars, int
 constexpr int kDiffLists = 256;
 struct DiffSink {
   unsigned long long* list;   // [kDiffLists * cap]
-  int32_t* count;             // [kDiffLists]
+  int32_t* count;             // [kDiffLists], then the propagators the base store does not satisfy
   int64_t cap;                // entries per sub-list
   int2* base;                 // [nvars]: the base store, written by the load
   int2* vals;                 // [kDiffLists * cap]: each entry's value (nullptr: not kept)
@@ -222,9 +222,10 @@ hipError_t launch_ingest_interleave(const int32_t* lb, const int32_t* ub, int2* 
                                     int64_t nvars, int64_t n_inst, int gi, uint8_t* empty,
                                     const DiffSink& ds, hipStream_t st);
 // The base store of device-resident lb / ub rows (rows 0-2) into ds.base,
-// before launch_ingest_rows lists the differences from it.
+// before launch_ingest_rows lists the differences from it; clears ds.count and
+// empty.
 hipError_t launch_make_base_rows(const int32_t* lb, const int32_t* ub, int64_t nvars, int64_t n_inst,
-                                 const DiffSink& ds, hipStream_t st);
+                                 const DiffSink& ds, uint8_t* empty, hipStream_t st);
 // Device-resident lb / ub into the stores only (no image copy), with the
 // differences from the base store (made first) and their values into ds,
 // and the emptiness; a complete list is the image (launch_image_from_diffs).
@@ -345,9 +346,11 @@ hipError_t launch_local(const Table& t, const LocalJob& job, int dom, int device
 hipError_t launch_adj_records(const Table& t, const int32_t* adj, int64_t n, int4* rec, hipStream_t st);
 // resident workgroups per CU (lds_bytes of dynamic LDS per workgroup)
 int persistent_blocks_per_cu(int dom, int64_t lds_bytes);
-// empty (may be nullptr): per-instance bytes, 1 = the store starts empty
+// empty (may be nullptr): per-instance bytes, 1 = the store starts empty; tight and
+// seed_n (may be nullptr): 2 * kTightSlots counters and n_inst counts to clear
 hipError_t launch_init_flags(InstFlags* flags, int32_t n_inst, WorkList wl, hipStream_t st,
-                             const uint8_t* empty = nullptr);
+                             const uint8_t* empty = nullptr, unsigned long long* tight = nullptr,
+                             int32_t* seed_n = nullptr);
 hipError_t launch_store_empty_map(const int2* store, int64_t nvars, int32_t n_inst, uint8_t* empty,
                                   int dom, hipStream_t st);
 hipError_t launch_schedule_slots(const SlotDesc* slots, InstFlags* flags, int32_t n_slots,

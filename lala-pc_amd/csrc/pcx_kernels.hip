@@ -2457,10 +2457,15 @@ hipError_t launch_persistent(const Table& t, int2* store, int64_t nvars, const S
 }
 
 // ---- bookkeeping kernels --------------------------------------------------
+// One launch for everything a run starts from zero: a clear of its own for the
+// counters and another for the lists' counts cost 5 to 10 us each, on the host or
+// between two kernels.
 __global__ void k_init_flags(InstFlags* flags, int32_t n_inst, WorkList wl,
-                             const uint8_t* __restrict__ empty) {
+                             const uint8_t* __restrict__ empty, unsigned long long* tight, int32_t* seed_n) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (tight && k < 2 * kTightSlots) tight[k] = 0;
   if (k < n_inst) {
+    if (seed_n) seed_n[k] = 0;
     flags[k].changed[0] = -2;
     flags[k].changed[1] = -1;      // "sweep -1 changed" lets sweep 0 run
     flags[k].failed_at = (empty && empty[k]) ? -1 : kNoFail;
@@ -2475,14 +2480,15 @@ __global__ void k_init_flags(InstFlags* flags, int32_t n_inst, WorkList wl,
     *wl.sweep = -1;
     *wl.n_act = 0;
     *wl.live = n_inst;
-    wl.live[1] = 0;                // persistent-mode queue head (ctl[3])
+    wl.live[1] = 0;                // queue head (ctl[3]) of a run that takes whole instances
   }
 }
 
 hipError_t launch_init_flags(InstFlags* flags, int32_t n_inst, WorkList wl, hipStream_t stream,
-                             const uint8_t* empty) {
+                             const uint8_t* empty, unsigned long long* tight, int32_t* seed_n) {
+  static_assert(2 * kTightSlots <= 256, "one workgroup clears the counters");
   const int grid = (int)((n_inst + 255) / 256);
-  k_init_flags<<<grid > 0 ? grid : 1, 256, 0, stream>>>(flags, n_inst, wl, empty);
+  k_init_flags<<<grid > 0 ? grid : 1, 256, 0, stream>>>(flags, n_inst, wl, empty, tight, seed_n);
   return hipGetLastError();
 }
 
@@ -2690,10 +2696,17 @@ hipError_t launch_branch_seed(const EventSet& ev, const int32_t* var, int64_t n_
 // batch of splits of one root.
 
 // The base store (base_value per variable) from rows 0-2 of lb / ub, or of
-// packed stores (lb == nullptr: rows of `store`).
+// packed stores (lb == nullptr: rows of `store`).  It also clears what the load's
+// pass over the stores counts in (empty [n_inst], ctl [kDiffLists + 1]), when given.
 __global__ __launch_bounds__(kBlock) void k_make_base(const int32_t* __restrict__ lb, const int32_t* __restrict__ ub,
                                                       const u64* __restrict__ store, int64_t nvars,
-                                                      int64_t n_inst, u64* __restrict__ base) {
+                                                      int64_t n_inst, u64* __restrict__ base,
+                                                      uint8_t* __restrict__ empty, int32_t* __restrict__ ctl) {
+  const int64_t at = (int64_t)blockIdx.x * kBlock + threadIdx.x, step = (int64_t)gridDim.x * kBlock;
+  if (empty)
+    for (int64_t k = at; k < n_inst; k += step) empty[k] = 0;
+  if (ctl)
+    for (int64_t c = at; c < kDiffLists + 1; c += step) ctl[c] = 0;
   for (int64_t v = (int64_t)blockIdx.x * kBlock + threadIdx.x; v < nvars; v += (int64_t)gridDim.x * kBlock) {
     auto row = [&](int64_t k) { return lb ? pack_bounds(lb[k * nvars + v], ub[k * nvars + v]) : store[k * nvars + v]; };
     const u64 a = row(0);
@@ -2701,10 +2714,11 @@ __global__ __launch_bounds__(kBlock) void k_make_base(const int32_t* __restrict_
   }
 }
 hipError_t launch_make_base(const int32_t* lb, const int32_t* ub, const u64* store, int64_t nvars,
-                            int64_t n_inst, u64* base, hipStream_t stream) {
+                            int64_t n_inst, u64* base, hipStream_t stream, uint8_t* empty = nullptr,
+                            int32_t* ctl = nullptr) {
   int64_t grid = (nvars + kBlock - 1) / kBlock;
   if (grid > 8192) grid = 8192;
-  k_make_base<<<(unsigned)grid, kBlock, 0, stream>>>(lb, ub, store, nvars, n_inst, base);
+  k_make_base<<<(unsigned)grid, kBlock, 0, stream>>>(lb, ub, store, nvars, n_inst, base, empty, ctl);
   return hipGetLastError();
 }
 
@@ -2886,9 +2900,10 @@ __global__ __launch_bounds__(kBlock) void k_ingest_held(const int32_t* __restric
 }
 
 hipError_t launch_make_base_rows(const int32_t* lb, const int32_t* ub, int64_t nvars, int64_t n_inst,
-                                 const DiffSink& ds, hipStream_t stream) {
-  if (!ds.list || nvars <= 0 || n_inst <= 0) return hipSuccess;
-  return launch_make_base(lb, ub, nullptr, nvars, n_inst, reinterpret_cast<u64*>(ds.base), stream);
+                                 const DiffSink& ds, uint8_t* empty, hipStream_t stream) {
+  if (!ds.list || nvars <= 0 || n_inst <= 0) return hipErrorInvalidValue;
+  return launch_make_base(lb, ub, nullptr, nvars, n_inst, reinterpret_cast<u64*>(ds.base), stream, empty,
+                          ds.count);
 }
 
 hipError_t launch_ingest_rows(const int32_t* lb, const int32_t* ub, int2* store, int64_t nvars,
@@ -3346,6 +3361,8 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
     if (k >= ev.n_inst) break;
     InstFlags* f = flags + k;
     uint32_t* row = ev.dirty + k * ev.words;           // plane 0: the seeds, and marks that overflow
+    if (ev.summary)                                    // a branching's seeds set bits there too
+      for (int64_t w = tid; w < ev.swords; w += B) ev.summary[k * ev.swords + w] = 0;
     if (f->failed_at != kNoFail) {                     // the same word for every thread: uniform
       for (int64_t w = tid; w < ev.words; w += B) row[w] = 0;   // its seeds: the row ends clear
       if (tid == 0 && trail.list) trail.n[k] = 0;

@@ -61,13 +61,6 @@ pcx_status scratch_of(int device, uint8_t** out) {
   return PCX_OK;
 }
 
-// Zeroes n 8-byte words (the tightening counters): a kernel, so the call
-// records no memset node if a caller captures its stream.
-__global__ void k_zero_u64(unsigned long long* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0ull;
-}
-
 }  // namespace
 
 extern "C" {
@@ -118,9 +111,7 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
 
   // Every value the sweeps read is written first: flags, counters, store.
   const WorkList wl = worklist_of(d_act, d_base, d_ctl);
-  PCX_HIP(launch_init_flags(d_flags, 1, wl, s));
-  k_zero_u64<<<1, 2 * kTightSlots, 0, s>>>(d_tight, 2 * kTightSlots);
-  PCX_HIP(hipGetLastError());
+  PCX_HIP(launch_init_flags(d_flags, 1, wl, s, nullptr, d_tight));
   PCX_HIP(launch_store_pack(d_lb, d_ub, d_store, nvars, s));
   PCX_HIP(launch_store_check_empty(d_store, nvars, 1, d_flags, dom, s));
 

@@ -942,12 +942,12 @@ pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, 
                                   b->d_unsat, n_unsat, seeds, e->stream));
   }
   if (drain) {
-    const int dgrid = (int)std::min<int64_t>(b->n_inst, (int64_t)pcx_internal::device_cus(e->cfg.device) * 24);
     pcx_status ts = tm.begin(e->stream);
     if (ts != PCX_OK) return ts;
     PCX_HIP(launch_drain_marks(table_of(e), b->d_store, b->nvars, b->d_flags, ev, b->d_ctl + 3,
                                b->d_tight + kTightSlots, seeds, InstLists{b->d_trail, b->d_trail_n, kTrailCap},
-                               b->image_absent ? b->d_undo : nullptr, b->d_image, dom_of(e), dgrid, e->stream));
+                               b->image_absent ? b->d_undo : nullptr, b->d_image, dom_of(e),
+                               pcx_internal::device_cus(e->cfg.device), e->stream));
     ts = tm.end(e->stream, false);
     if (ts != PCX_OK) return ts;
     std::vector<InstFlags> flags;

@@ -272,7 +272,7 @@ hipError_t launch_seed_from_base(const EventSet& ev, const DiffSink& diffs, int6
 // restore rewrites only those.
 hipError_t launch_drain_marks(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
                               int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
-                              const InstLists& trail, int2* undo, int2* image, int dom, int grid, hipStream_t st);
+                              const InstLists& trail, int2* undo, int2* image, int dom, int cus, hipStream_t st);
 // A drain with undo ([n_inst * trail.cap] values) also lists, beside each variable
 // of the trail, the value it was tightened from, and writes an instance's row of
 // image before its trail overflows.  launch_undo: dst (the stores, or the image)

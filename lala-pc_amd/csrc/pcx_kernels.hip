@@ -3268,16 +3268,17 @@ __device__ __forceinline__ void drain_list(int32_t q, uint32_t* row, int32_t* hs
   *over = 1;
 }
 
-// The member propagators adjacent to v, listed for the next round; eight
-// adjacency entries (and their member words) in flight at a time.
-__device__ __forceinline__ void drain_mark(uint32_t* row, const uint32_t* mrow, const EventSet& ev, int32_t v,
-                                           int32_t* hs, int32_t* list, int32_t* n, int32_t* over) {
+// The member propagators adjacent to v, listed for the next round, by the g
+// threads of a group (this one is its l-th); eight adjacency entries (and their
+// member words) of a thread in flight at a time.
+__device__ __forceinline__ void drain_mark(uint32_t* row, const uint32_t* mrow, const EventSet& ev, int32_t v, int l,
+                                           int g, int32_t* hs, int32_t* list, int32_t* n, int32_t* over) {
   constexpr int kB = 8;
   const int32_t e = ev.adj_off[v + 1];
-  for (int32_t i = ev.adj_off[v]; i < e; i += kB) {
+  for (int32_t i = ev.adj_off[v] + l; i < e; i += kB * g) {
     int32_t q[kB];
 #pragma unroll
-    for (int j = 0; j < kB; ++j) q[j] = i + j < e ? ev.adj[i + j] : -1;
+    for (int j = 0; j < kB; ++j) q[j] = i + j * g < e ? ev.adj[i + j * g] : -1;
     uint32_t in[kB];
 #pragma unroll
     for (int j = 0; j < kB; ++j) in[j] = (q[j] >= 0 && mrow) ? mrow[q[j] >> 5] : ~0u;
@@ -3464,17 +3465,24 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
             s_tv[at] = vs[j];
             if (UNDO) s_old[at] = ws[j];
           } else {
-            drain_mark(row, mrow, ev, vs[j], s_hash, s_list[nx], &s_n[nx], &s_over[nx]);
+            drain_mark(row, mrow, ev, vs[j], 0, 1, s_hash, s_list[nx], &s_n[nx], &s_over[nx]);
             on_trail(vs[j], ws[j]);
           }
         }
       }
       __syncthreads();                                 // the round's tightened variables are listed
-      // (C) list their adjacency, a variable per thread
+      // (C) list their adjacency, a variable per group of threads: the largest
+      // groups that take every variable at once.  A round tightens few variables
+      // (45 in seven rounds of a slow instance) of a dozen or more propagators each:
+      // one thread a variable left the others idle behind a chain of three loads per
+      // eight propagators, 12 us of a round's 17; 4,096 instances of 50,000 variables
+      // took 219 us so and take 147.
       const int ntv = min(s_ntv, kDrainVars);
-      for (int i = tid; i < ntv; i += B) {
-        drain_mark(row, mrow, ev, s_tv[i], s_hash, s_list[nx], &s_n[nx], &s_over[nx]);
-        on_trail(s_tv[i], UNDO ? s_old[i] : 0);
+      int g = kWave;
+      while (g > 1 && ntv * g > B) g >>= 1;
+      for (int i = tid / g; i < ntv; i += B / g) {
+        drain_mark(row, mrow, ev, s_tv[i], tid & (g - 1), g, s_hash, s_list[nx], &s_n[nx], &s_over[nx]);
+        if ((tid & (g - 1)) == 0) on_trail(s_tv[i], UNDO ? s_old[i] : 0);
       }
       if (__ballot(chg) && lane_id() == 0) s_chg = 1;
       if (__ballot(fail) && lane_id() == 0) s_fail = 1;
@@ -3500,18 +3508,12 @@ __global__ __launch_bounds__(B) void k_drain_marks(Table t, int2* __restrict__ s
 }
 
 namespace {
-template <bool UNDO>
-hipError_t launch_drain_u(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
+template <int B, bool UNDO>
+hipError_t launch_drain_b(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
                           int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
-                          const InstLists& trail, u64* undo, u64* image, int dom, int grid, hipStream_t stream) {
-  // Workgroups of two waves: at 4,096 interval instances of 50,000 variables
-  // 0.228 ms against 0.236 with one wave and 0.255 with four (the replayed
-  // step 0.33 ms against 0.35-0.36); at 1,024 bitset instances of 200,000
-  // words 98 us against 105 with one wave.
-  constexpr int kDrainB = 2 * kWave;
+                          const InstLists& trail, u64* undo, u64* image, int dom, unsigned grid, hipStream_t stream) {
 #define PCX_DRAIN(D) \
-  k_drain_marks<D, kDrainB, UNDO><<<grid, kDrainB, 0, stream>>>(t, store, nvars, flags, ev, next_inst, tight, seeds, \
-                                                                trail, undo, image)
+  k_drain_marks<D, B, UNDO><<<grid, B, 0, stream>>>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail, undo, image)
   switch (dom) {
     case kItv: PCX_DRAIN(kItv); break;
     case kItvDiv: PCX_DRAIN(kItvDiv); break;
@@ -3525,12 +3527,22 @@ hipError_t launch_drain_u(const Table& t, int2* store, int64_t nvars, InstFlags*
 
 hipError_t launch_drain_marks(const Table& t, int2* store, int64_t nvars, InstFlags* flags, const EventSet& ev,
                               int32_t* next_inst, unsigned long long* tight, const InstLists& seeds,
-                              const InstLists& trail, int2* undo, int2* image, int dom, int grid, hipStream_t stream) {
+                              const InstLists& trail, int2* undo, int2* image, int dom, int cus, hipStream_t stream) {
   if (ev.n_inst <= 0 || !ev.dirty) return hipSuccess;
   if (undo && (!image || !trail.list)) return hipErrorInvalidValue;
   u64 *u = reinterpret_cast<u64*>(undo), *im = reinterpret_cast<u64*>(image);
-  return undo ? launch_drain_u<true>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail, u, im, dom, grid, stream)
-              : launch_drain_u<false>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail, u, im, dom, grid, stream);
+  // Workgroups of four waves while they are all resident (eight on a compute
+  // unit), else of two: 2,048 children of 50,000 variables take 58 us against 64
+  // with two waves, 64 bitset instances 49 against 56, but 4,096 instances 155
+  // against 147 (195 with one wave).
+  constexpr int kNarrow = 2 * kWave, kWide = 4 * kWave;
+  const bool wide = ev.n_inst <= (int64_t)cus * 8;
+  const unsigned grid = (unsigned)(ev.n_inst < (int64_t)cus * 24 ? ev.n_inst : (int64_t)cus * 24);
+#define PCX_DRAIN_B(B, U) \
+  launch_drain_b<B, U>(t, store, nvars, flags, ev, next_inst, tight, seeds, trail, u, im, dom, grid, stream)
+  if (undo) return wide ? PCX_DRAIN_B(kWide, true) : PCX_DRAIN_B(kNarrow, true);
+  return wide ? PCX_DRAIN_B(kWide, false) : PCX_DRAIN_B(kNarrow, false);
+#undef PCX_DRAIN_B
 }
 
 hipError_t launch_seed_from_base(const EventSet& ev, const DiffSink& diffs, int64_t n_diffs,

@@ -127,3 +127,34 @@ def test_children_keep_their_image(gpu, bits, shape):
     assert _same(_read(bits, grand), below)
     child.reset()
     assert _same(_read(bits, child), children)
+
+
+@pytest.mark.parametrize("n", [3, 1020, 1050], ids=["few", "wide", "narrow"])
+@pytest.mark.parametrize("fan", [1, 2, 3, 7, 31, 64, 65, 130, 300])
+def test_rounds_of_any_width(gpu, n, fan):
+    """A drained round that tightens `fan` variables at once, whose adjacency lists groups of
+    64 threads down to one walk (and, past 256 variables, the evaluating threads), one variable
+    of them a hub with more propagators than a group has threads; workgroups of both widths."""
+    hub = 90
+    V = 1 + fan + fan + hub + 1
+    zero = V - 1
+    x = np.concatenate([1 + np.arange(fan), 1 + fan + np.arange(fan), 1 + 2 * fan + np.arange(hub)]).astype(np.int32)
+    y = np.concatenate([np.zeros(fan), 1 + np.arange(fan), np.full(hub, 1)]).astype(np.int32)
+    z = np.full(len(x), zero, np.int32)
+    lo, hi = np.zeros(V, np.int32), np.full(V, 9, np.int32)
+    hi[zero] = 0
+    pir = pcx.PIR()
+    pir.tell(np.full(len(x), ol.OPS["ADD"], np.int32), x, y, z, lo, hi)
+    lb, ub = np.tile(lo, (n, 1)), np.tile(hi, (n, 1))
+    lb[:, 0] = np.random.default_rng(fan).integers(0, 9, n)
+    parent = pcx.Batch(pir, n, V)
+    parent.load(lb.reshape(-1), ub.reshape(-1))
+    parent.run(pcx.MODE_BATCHED)
+    child = pcx.Batch(pir, 2 * n, V)
+    parent.branch(child, from_fixpoint=True)
+    ref = [a.copy() for a in child.read()]
+    rg, st = child.run(pcx.MODE_BATCHED)
+    assert st.full_evals == 0                    # drained
+    ro = ol.fixpoint_batch(*pir.table(), ref[0], ref[1], V)
+    assert [r.failed for r in rg] == [r.failed for r in ro]
+    assert _same(list(child.read()), ref)

@@ -495,9 +495,11 @@ pcx_status prepare_events(pcx_batch* b, int32_t mode) {
 
 EventSet event_set(const pcx_batch* b) {
   const int64_t srows = b->n_inst * summary_words(b);
-  return EventSet{b->e->d_adj_off, b->e->d_adj, b->h_off.empty() ? nullptr : b->d_member,
-                  b->d_dirty, b->d_summary, b->d_summary ? b->d_summary + 2 * srows : nullptr,
-                  bitmap_words(b), summary_words(b), b->n_inst};
+  EventSet ev{b->e->d_adj_off, b->e->d_adj, b->h_off.empty() ? nullptr : b->d_member,
+              b->d_dirty, b->d_summary, b->d_summary ? b->d_summary + 2 * srows : nullptr,
+              bitmap_words(b), summary_words(b), b->n_inst};
+  ev.adj_vars = (int32_t)b->e->adj_vars;
+  return ev;
 }
 
 // Table and subsets a sweep kernel reads for this batch.

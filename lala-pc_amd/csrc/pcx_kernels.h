@@ -64,8 +64,8 @@ struct InstFlags {
 constexpr int kChunkWords = 256;
 constexpr int kChunkShift = 13;            // propagators per chunk = 1 << 13
 struct EventSet {
-  const int32_t* adj_off;   // [nvars + 1]
-  const int32_t* adj;       // [adj_off[nvars]]
+  const int32_t* adj_off;   // [adj_vars + 1]
+  const int32_t* adj;       // [adj_off[adj_vars]]
   const uint32_t* member;   // [n_inst * words] or nullptr
   uint32_t* dirty;          // [2 * n_inst * words], or nullptr = no marking
   uint32_t* summary;        // [2 * n_inst * swords]
@@ -86,6 +86,9 @@ struct EventSet {
   unsigned long long* q;    // [2 * kQLists * qcap]
   int32_t* qctl;
   int64_t qcap;             // entries per sub-list
+  // Variables with adjacency offsets: up to the last one the table names.  A store
+  // may hold more, which no propagator tightens but a load or a split may change.
+  int32_t adj_vars;
 };
 constexpr int kQLists = 256;
 // Queue control words.

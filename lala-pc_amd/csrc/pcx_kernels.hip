@@ -2667,7 +2667,7 @@ __global__ __launch_bounds__(kBlock) void k_branch_seed(EventSet ev, const int32
                                                         int64_t n_child) {
   for (int64_t c = blockIdx.x; c < n_child; c += gridDim.x) {
     const int32_t v = var[c >> 1];
-    if (v < 0) continue;                          // uniform: no split, no marks
+    if (v < 0 || v >= ev.adj_vars) continue;      // uniform: no split, or of a variable no propagator reads
     Marker mk = marker_for(&ev, c, -1);           // sweep -1 marks plane 0 (sweep 0's)
     for (int32_t i = ev.adj_off[v] + threadIdx.x; i < ev.adj_off[v + 1]; i += kBlock) {
       const int32_t p = ev.adj[i];
@@ -3207,8 +3207,9 @@ __global__ __launch_bounds__(kBlock) void k_seed_from_base(EventSet ev, DiffSink
         const int64_t k = (int64_t)(d >> 32);
         const int32_t v = (int32_t)(uint32_t)d;
         const Marker mk = marker_for(&ev, k, -1);          // sweep -1 marks plane 0 (sweep 0's)
-        for (int32_t a = ev.adj_off[v] + (threadIdx.x & 3); a < ev.adj_off[v + 1]; a += 4)
-          seed_prop(mk, ev, qs, sl, k, ev.adj[a]);
+        if (v < ev.adj_vars)                               // else no propagator reads it
+          for (int32_t a = ev.adj_off[v] + (threadIdx.x & 3); a < ev.adj_off[v + 1]; a += 4)
+            seed_prop(mk, ev, qs, sl, k, ev.adj[a]);
       }
     } else {
       const int64_t j = (it - diff_steps) * kBlock + threadIdx.x;

@@ -74,9 +74,11 @@ typedef struct {
   int32_t props_per_wave;   /* 64 .. 512 (powers of two; batched mode also 1024 and
                                2048: work items of 2 or 4 rounds of 512); 0 = chosen
                                from the sweep size                                   */
-  int32_t lds_mode;         /* persistent mode: stage each store in LDS; 0 never,
-                               1 or -1 (auto) whenever it fits in a workgroup's
-                               LDS (160 KB on MI355X)                              */
+  int32_t lds_mode;         /* stage small stores in LDS; 0 never, 1 or -1 (auto)
+                               whenever a store fits in a workgroup's LDS (160 KB
+                               on MI355X): every persistent run, small single
+                               stores, and batched interval runs that the
+                               automatic settings leave unseeded                    */
   int32_t sweeps_per_check; /* plain engine: sweeps queued between host checks (0=8) */
   int64_t max_sweeps;       /* 0 = run to the fixpoint                               */
   int32_t timing;           /* 1 = record HIP events around every sweep kernel       */
@@ -86,10 +88,13 @@ typedef struct {
                                own copy of its subset (12 B per active propagator)  */
   int32_t stream_tables;    /* -1 auto (stream per-instance tables only), 0 cached
                                table loads, 1 non-temporal table loads               */
-  int32_t event_driven;     /* -1 auto (batched mode; plain mode from 2^20
-                               propagators per instance), 0 every sweep evaluates
-                               every propagator, 1 sweeps after the first evaluate
-                               only propagators with an operand tightened since     */
+  int32_t event_driven;     /* 0 every sweep evaluates every propagator, 1 sweeps
+                               after the first evaluate only propagators with an
+                               operand tightened since, -1 auto (batched mode and
+                               LDS runs do; plain runs of one whole-table store
+                               follow the operands they tighten instead, in
+                               launches that start as full sweeps; of several
+                               stores or subsets, from 2^20 propagators)            */
   int32_t lockstep;         /* batched mode, full sweeps: 0 per-instance work items;
                                16, 32 or 64: one propagator for that many instances
                                per step, over an instance-interleaved copy of the
@@ -197,8 +202,10 @@ pcx_status pcx_fixpoint(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars,
  * in one fixed device array of the library per GPU, which holds stores of
  * at most PCX_NOALLOC_MAX_VARS variables (PCX_EINVAL beyond that), and the
  * engine's table must fit its device copy (after a tell that grew the
- * table, one pcx_fixpoint call sizes it; PCX_EINVAL otherwise).  Sweeps are
- * full sweeps (no marks, which would need memory per propagator); the
+ * table, one pcx_fixpoint call sizes it; PCX_EINVAL otherwise).  Where an
+ * earlier pcx_fixpoint on this table built its adjacency, the call runs as
+ * pcx_fixpoint does (a small store in LDS, a large one chasing what it
+ * tightens); otherwise sweeps are full sweeps.  The
  * fixpoint is the one pcx_fixpoint gives.  Calls that overlap on one GPU
  * share that array and race: one call at a time per GPU. */
 #define PCX_NOALLOC_MAX_VARS (1 << 21)
@@ -240,8 +247,8 @@ pcx_status pcx_batch_load_device(pcx_batch* b, const int32_t* d_lb, const int32_
 /* PC's is_extractable on every store of the batch (pc.hpp:727-738: the
  * store is not empty and every formula is asked), for formula trees in the
  * postorder node form of pcx_model.h (nodes: 4 * n_nodes int32, off:
- * n_formulas + 1 offsets; pcx_model_formulas gives a model's trees).  One
- * GPU thread per (store, formula) interprets its tree.  extractable[k] is
+ * n_formulas + 1 offsets; pcx_model_formulas gives a model's trees).  A GPU
+ * lane per (store, formula) interprets its tree.  extractable[k] is
  * 1 or 0.  Errors: PCX_EINVAL for a malformed tree (unknown kind, a variable
  * outside the store, a stack deeper than 32 or left with more than one
  * value).  Interval batches. */

@@ -21,7 +21,8 @@ struct pcx_engine {
   uint64_t adj_version = 0;
   int64_t adj_vars = 0;               // variables with offsets (max_var + 1 then)
   int64_t adj_n = 0;                  // adjacency entries
-  int4* d_adj_rec = nullptr;          // the adjacency with table entries (LDS kernel), on demand
+  int4* d_adj_rec = nullptr;          // the adjacency with table entries (the LDS
+                                      // kernel and the chase), on demand
   uint64_t adj_rec_version = 0;
   uint32_t* d_xo = nullptr;
   int32_t* d_y = nullptr;

@@ -1537,6 +1537,15 @@ pcx_status pcx_batch_load_device(pcx_batch* b, const int32_t* d_lb, const int32_
   pcx_engine* e = b->e;
   PCX_HIP(hipSetDevice(e->cfg.device));
   const int64_t n = b->n_inst * b->nvars;
+  const int gi = lockstep_of(b);
+  // A load that still has to allocate may fail with the stores half written: an
+  // image that lies in them is written out first.
+  const bool allocates = !b->d_diff || !b->d_unsat ||
+                         (gi > 0 && b->shadow_words < (b->n_inst + gi - 1) / gi * gi * b->nvars);
+  if (b->image_absent && allocates && (b->store_is_image || b->trail_valid)) {
+    pcx_status st = write_absent_image(b);
+    if (st != PCX_OK) return st;
+  }
   // Stores that hold their image as a base store plus a complete difference
   // list (or that image but for the trail of a drained run from it) go back
   // to the base store first: the ingest then writes only the values that
@@ -1559,7 +1568,6 @@ pcx_status pcx_batch_load_device(pcx_batch* b, const int32_t* d_lb, const int32_
   DiffSink ds;
   pcx_status dst = diff_sink(b, &ds, !b->shared_loads);
   if (dst != PCX_OK) return dst;
-  const int gi = lockstep_of(b);
   const bool rows = ds.list && b->shared_loads;
   if (rows) PCX_HIP(launch_make_base_rows(d_lb, d_ub, b->nvars, b->n_inst, ds, b->d_image_empty, e->stream));
   else PCX_HIP(hipMemsetAsync(b->d_image_empty, 0, b->n_inst, e->stream));

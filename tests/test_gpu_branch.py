@@ -158,3 +158,30 @@ def test_rounds_of_any_width(gpu, n, fan):
     ro = ol.fixpoint_batch(*pir.table(), ref[0], ref[1], V)
     assert [r.failed for r in rg] == [r.failed for r in ro]
     assert _same(list(child.read()), ref)
+
+
+@pytest.mark.parametrize("ran", [False, True], ids=["branched", "drained"])
+@pytest.mark.parametrize("gi", [0, 16])
+def test_children_are_loaded_over(gpu, gi, ran):
+    """Stores loaded from device memory into children that hold no image are the new image."""
+    from pcx.device import DeviceArray
+    pir, V, (lo, hi) = _net(False, 1100, 7)
+    pir.set_config(lockstep=gi)
+    n = 3
+    parent, child = pcx.Batch(pir, n, V), pcx.Batch(pir, 2 * n, V)
+    parent.load(np.tile(lo, n), np.tile(hi, n))
+    parent.run(pcx.MODE_BATCHED)
+    lb, ub = np.tile(lo, 2 * n), np.tile(hi, 2 * n)
+    lb[V], ub[4 * V] = 2, 5
+    want, res = _oracle(False, pir, [lb, ub], V)
+    dev = [DeviceArray(lb), DeviceArray(ub)]
+    for _ in range(2):                           # (the second load finds its lists there)
+        parent.branch(child, from_fixpoint=True)
+        if ran:
+            child.run(pcx.MODE_BATCHED)
+        child.load_device(dev[0].ptr, dev[1].ptr)
+        rg, _ = child.run(pcx.MODE_BATCHED)
+        assert [r.failed for r in rg] == [r.failed for r in res]
+        assert _same(list(child.read()), want)
+        child.reset()
+        assert _same(list(child.read()), [lb, ub])

@@ -101,6 +101,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
   constexpr int kStack = kLocalList / kWaves;        // marks on a wave's stack: its share of a list
   extern __shared__ u64 s_dyn[];
   __shared__ int32_t s_slot, s_fail, s_chg, s_steps;
+  __shared__ int32_t s_empty;                        // empty as loaded: no round writes it, a late wave may still read it
   __shared__ int32_t s_ntv[2], s_n[2], s_over[2];    // by parity of the round
   __shared__ int32_t s_sum[3];
   const int tid = threadIdx.x, lane = lane_id(), wave = uni(tid / kWave);
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       if (mrow) return mrow[w];
       return (w == W - 1 && (P & 31)) ? (1u << (P & 31)) - 1u : ~0u;
     };
-    if (tid == 0) { s_fail = 0; s_chg = 0; s_steps = 0; s_ntv[0] = s_ntv[1] = 0; s_n[0] = s_n[1] = 0; s_over[0] = 1; s_over[1] = 0; }
+    if (tid == 0) { s_fail = 0; s_empty = 0; s_chg = 0; s_steps = 0; s_ntv[0] = s_ntv[1] = 0; s_n[0] = s_n[1] = 0; s_over[0] = 1; s_over[1] = 0; }
     if (tid < 3) s_sum[tid] = 0;
     __syncthreads();                                 // s_slot is read; the counters are set
     if (!start_failed) {
@@ -152,9 +153,9 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       }
       for (int32_t w = tid; w < W; w += B) bm[w] = member_word(w);
       for (int32_t w = tid; w < VW; w += B) vbm[w] = 0;
-      if (empty) s_fail = 1;
+      if (empty) s_empty = 1;
       __syncthreads();
-      start_failed = s_fail != 0;
+      start_failed = s_empty != 0;
     }
 
     int32_t failed_at = start_failed ? -1 : kNoFail, r = 0;

@@ -15,6 +15,10 @@
 // workgroups tighten them during the launch.  Neighbours that find the ring full are dropped: a sweep that
 // tightened anything is followed by another one over the whole table, and only a
 // sweep that tightened nothing -- which read one constant store -- ends the run.
+// For the same reason a wave may stop: after kChaseLinks links of a launch it drops
+// what it was chasing and only evaluates the rest of its propagators once, so that
+// a launch ends (after about 10 ms of links) however slowly the store converges,
+// and a store that another wave has failed is left within kChaseLook links.
 //
 // What bounds it: three dependent trips to memory a link (operands; meets;
 // adjacency records; about 2.3 us together), and the longest chain of links.  It
@@ -36,6 +40,8 @@ constexpr int kChaseWaves = kBlock / kWave;
 constexpr int kChaseRing = 1024;       // records' positions waiting, per wave (a power of two)
 constexpr int kChaseLanes = 8;          // lanes that walk one variable's adjacency
 constexpr int kChaseVars = kWave / kChaseLanes;
+constexpr int kChaseLinks = 4096;       // links a wave chases in one launch
+constexpr int kChaseLook = 16;          // links between two looks at the store's failure (a power of two)
 
 }  // namespace
 
@@ -57,7 +63,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep_chase(Table t, int2* st, int32
   };
   const int64_t n_waves = (int64_t)gridDim.x * kChaseWaves;
   bool chg = false, fail = false;
-  int nt = 0, ne = 0;
+  int nt = 0, ne = 0, links = 0;
   for (int64_t base = ((int64_t)blockIdx.x * kChaseWaves + wave) * kWave; base < t.n; base += n_waves * kWave) {
     uint32_t head = 0, tail = 0;                     // the ring's entries, the same in every lane
     bool on = base + lane < t.n;
@@ -111,6 +117,10 @@ __global__ __launch_bounds__(kBlock) void k_sweep_chase(Table t, int2* st, int32
       const unsigned long long mx = __ballot(tx), my = __ballot(ty), mz = __ballot(tz);
       chg |= (mx | my | mz) != 0;
       if (__ballot(fail)) break;
+      if (!first && ((++links & (kChaseLook - 1)) == 0) &&
+          __hip_atomic_load(&f->failed_at, __ATOMIC_RELAXED, AG) != kNoFail)
+        break;
+      if (links >= kChaseLinks) break;
       const int cx = __builtin_popcountll(mx), cy = cx + __builtin_popcountll(my);
       const int nv = cy + __builtin_popcountll(mz);
       if (tx) walk[below(mx)] = ax;

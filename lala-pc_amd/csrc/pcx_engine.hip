@@ -145,8 +145,10 @@ bool single_local(const pcx_engine* e, int64_t nvars) {
 // The LDS kernel on one store of separate bounds, in memory the device can
 // address; flags may be pinned host memory.  The table and its adjacency
 // records are on the device.
-hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, InstFlags* flags) {
+hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, InstFlags* flags,
+                         bool resume) {
   LocalJob job{};
+  job.resume = resume;
   job.lb = lb;
   job.ub = ub;
   job.nvars = nvars;
@@ -652,12 +654,11 @@ pcx_status prepare_run(pcx_batch* b, int32_t mode, SeedPlan* plan, bool* local) 
   return prepare_events(b, mode);
 }
 
-// The LDS kernel over the batch: one launch, one workgroup per instance.
+// The LDS kernel over the batch: one launch, one workgroup per instance, and
+// further ones while it left instances unsettled.
 pcx_status run_local(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
   pcx_engine* e = b->e;
   SweepTimer tm{b, e->cfg.timing != 0};
-  pcx_status ts = tm.begin(e->stream);
-  if (ts != PCX_OK) return ts;
   LocalJob job{};
   job.store = b->d_store;
   job.nvars = b->nvars;
@@ -671,12 +672,21 @@ pcx_status run_local(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
   job.adj = e->d_adj_rec;
   job.member = b->h_off.empty() ? nullptr : b->d_member;
   job.words = bitmap_words(b);
-  PCX_HIP(launch_local(table_of(e), job, dom_of(e), e->cfg.device,
-                       pcx_internal::device_cus(e->cfg.device), e->stream));
-  ts = tm.end(e->stream, true);
-  if (ts != PCX_OK) return ts;
   std::vector<InstFlags> flags;
-  return collect(b, flags, results, stats, tm);
+  const double load_ms = b->load_ms;        // (collect hands it out once)
+  for (;;) {
+    pcx_status ts = tm.begin(e->stream);
+    if (ts != PCX_OK) return ts;
+    PCX_HIP(launch_local(table_of(e), job, dom_of(e), e->cfg.device,
+                         pcx_internal::device_cus(e->cfg.device), e->stream));
+    ts = tm.end(e->stream, true);
+    if (ts != PCX_OK) return ts;
+    b->load_ms = load_ms;
+    ts = collect(b, flags, results, stats, tm);
+    if (ts != PCX_OK || std::none_of(flags.begin(), flags.end(), local_unsettled)) return ts;
+    job.resume = true;
+    PCX_HIP(hipMemsetAsync(job.queue, 0, sizeof(int32_t), e->stream));
+  }
 }
 
 // Queue planes of a batch (queued marked sweeps), allocated on first use:
@@ -2068,8 +2078,12 @@ pcx_status fixpoint_local(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars
   int32_t* pub = plb + nvars;
   std::memcpy(plb, lb, nvars * sizeof(int32_t));
   std::memcpy(pub, ub, nvars * sizeof(int32_t));
-  PCX_HIP(pcx_internal::launch_single(e, plb, pub, nvars, flags));
-  PCX_HIP(hipStreamSynchronize(e->stream));
+  bool resume = false;
+  do {
+    PCX_HIP(pcx_internal::launch_single(e, plb, pub, nvars, flags, resume));
+    PCX_HIP(hipStreamSynchronize(e->stream));
+    resume = true;
+  } while (local_unsettled(*flags));
   std::memcpy(lb, plb, nvars * sizeof(int32_t));
   std::memcpy(ub, pub, nvars * sizeof(int32_t));
   if (out) *out = pcx_internal::single_result(e, *flags);

@@ -150,7 +150,8 @@ pcx_status ensure_adjacency(pcx_engine* e);   // variable -> table positions, on
 pcx_status ensure_adj_records(pcx_engine* e); // the same with each propagator's table entry
 // one small store through the LDS kernel (see pcx_engine.hip)
 bool single_local(const pcx_engine* e, int64_t nvars);
-hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx::InstFlags* flags);
+hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx::InstFlags* flags,
+                         bool resume);
 bool chase_wanted(const pcx_engine* e);       // plain runs of one store chase
 constexpr int kChaseAfter = 4;                // plain sweeps before the first chase (see pcx_chase.hip)
 pcx_result single_result(const pcx_engine* e, const pcx::InstFlags& f);

@@ -323,9 +323,11 @@ hipError_t launch_sweep_chase(const Table& t, int2* store, int32_t sweep, InstFl
 // workgroup per instance (pcx_local.hip).  Instances come either from a
 // batch's stores (store, n_inst slices; flags already initialised, an instance
 // with failed_at set is left alone; taken in `order` from *queue, zeroed by
-// the caller) or from one pair of bound arrays (lb / ub, one instance, which
+// the caller before each launch) or from one pair of bound arrays (lb / ub, one instance, which
 // the kernel reads and writes in place: memory the device can address,
 // emptiness found by the kernel, flags written whole).
+// A launch is bounded: instances that it leaves without a failure and unsettled
+// (local_unsettled) need another launch with resume set.
 struct LocalJob {
   int32_t* lb;              // or nullptr
   int32_t* ub;
@@ -341,7 +343,9 @@ struct LocalJob {
   const int4* adj;          // adjacency records (launch_adj_records)
   const uint32_t* member;   // [n_inst * words], or nullptr: every propagator
   int64_t words;
+  bool resume;              // go on from the stores and flags of the last launch
 };
+inline bool local_unsettled(const InstFlags& f) { return f.failed_at == kNoFail && f.settled_at < 0; }
 // whether a store and a table fit (store, bitmaps and lists in LDS)
 bool local_fits(int device, int64_t nvars, int64_t n_props);
 hipError_t launch_local(const Table& t, const LocalJob& job, int dom, int device, int cus, hipStream_t st);

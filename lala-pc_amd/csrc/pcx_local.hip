@@ -31,6 +31,12 @@
 // set knows that its holder has not read the operands yet.  When no bit is set,
 // every propagator was evaluated on operands that have not changed since.
 //
+// A launch gives an instance kLocalLinks rounds and chase steps.  One that is not
+// at its fixpoint then stays unsettled (settled_at < 0), its store as far as it
+// came, and the host launches again: the instance goes on with every propagator
+// marked, and its counts with it.  So a launch ends (in about 10 ms an instance)
+// however slowly a store converges.
+//
 // What bounds it: the depth of the propagation times the latency of one link
 // (operands and meets in LDS, the adjacency from L2, and the instructions of one
 // evaluation, which a lone wave issues one by one).
@@ -49,7 +55,9 @@ constexpr int kLocalList = 2048;       // propagators listed per round
 constexpr int kWalkLanes = 16;         // lanes that walk one variable's adjacency in a chase
 constexpr int kWalkVars = kWave / kWalkLanes;
 constexpr int kChasePerWave = 8;         // marks a wave chases at most when a chase starts
+constexpr int kLocalLinks = 4096;      // rounds and chase steps of an instance in one launch
 constexpr int64_t kLocalStatic = 256;  // static LDS of the kernel (counters), at most
+constexpr int32_t kResumeMax = 1 << 30;  // rounds a resumed run is taken to have had, at most (they are counted in 32 bits)
 
 // Workgroups of 1,024 threads (batches that leave compute units idle: the
 // dense rounds are then as wide as one unit allows) or 256 (larger batches:
@@ -89,6 +97,14 @@ hipError_t launch_adj_records(const Table& t, const int32_t* adj, int64_t n, int
   return hipGetLastError();
 }
 
+namespace {
+__device__ __forceinline__ long long wave_sum64(long long v) {
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+  return v;
+}
+}  // namespace
+
 template <int D, int B>
 constexpr int local_min_waves() { return B == kNarrow && D != kItvDiv ? 6 : 1; }
 
@@ -103,7 +119,8 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
   __shared__ int32_t s_slot, s_fail, s_chg, s_steps;
   __shared__ int32_t s_empty;                        // empty as loaded: no round writes it, a late wave may still read it
   __shared__ int32_t s_ntv[2], s_n[2], s_over[2];    // by parity of the round
-  __shared__ int32_t s_sum[3];
+  __shared__ int32_t s_out;                          // a wave ran out of steps
+  __shared__ unsigned long long s_sum[3];
   const int tid = threadIdx.x, lane = lane_id(), wave = uni(tid / kWave);
   const int32_t V = (int32_t)job.nvars, P = (int32_t)t.n;
   const int32_t W = (P + 31) >> 5, VW = (V + 31) >> 5;
@@ -130,14 +147,16 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
     const int32_t k = job.order ? job.order[slot] : slot;
     InstFlags* const f = job.flags + k;
     const bool soa = job.lb != nullptr;
-    bool start_failed = !soa && f->failed_at != kNoFail;
+    // (settled in an earlier launch of a run that goes on: nothing is left to do)
+    bool start_failed = !soa && (f->failed_at != kNoFail || (job.resume && f->settled_at >= 0));
+    const int32_t r0 = job.resume ? uni(min(max(f->done_at, 0), kResumeMax)) : 0;
     const uint32_t* const mrow = job.member ? job.member + (int64_t)k * job.words : nullptr;
     u64* const gst = soa ? nullptr : reinterpret_cast<u64*>(job.store) + (int64_t)k * V;
     auto member_word = [&](int32_t w) {              // every propagator of the instance
       if (mrow) return mrow[w];
       return (w == W - 1 && (P & 31)) ? (1u << (P & 31)) - 1u : ~0u;
     };
-    if (tid == 0) { s_fail = 0; s_empty = 0; s_chg = 0; s_steps = 0; s_ntv[0] = s_ntv[1] = 0; s_n[0] = s_n[1] = 0; s_over[0] = 1; s_over[1] = 0; }
+    if (tid == 0) { s_fail = 0; s_empty = 0; s_chg = 0; s_steps = 0; s_ntv[0] = s_ntv[1] = 0; s_n[0] = s_n[1] = 0; s_over[r0 & 1] = 1; s_over[(r0 & 1) ^ 1] = 0; s_out = 0; }
     if (tid < 3) s_sum[tid] = 0;
     __syncthreads();                                 // s_slot is read; the counters are set
     if (!start_failed) {
@@ -158,8 +177,9 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       start_failed = s_empty != 0;
     }
 
-    int32_t failed_at = start_failed ? -1 : kNoFail, r = 0;
-    int nt0 = 0, nt = 0;
+    int32_t failed_at = start_failed ? -1 : kNoFail, r = r0;
+    bool unsettled = false;
+    int nt0 = 0, nt = 0;                             // (a launch's share fits: kLocalLinks bounds it)
     int ne = 0;                                      // evaluations after round 0
     // Evaluate one propagator on the LDS store; which operands it tightened.
     bool fail = false;
@@ -192,6 +212,8 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       return !(__hip_atomic_fetch_or(&bm[q >> 5], bit, __ATOMIC_RELAXED, WG) & bit);
     };
     while (!start_failed) {
+      unsettled = r - r0 >= kLocalLinks;
+      if (unsettled) break;
       // ---- round r: (B)
       const int cur = r & 1, nx = cur ^ 1;
       PT* const list = lists + cur * kLocalList;
@@ -307,7 +329,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
           z = t.z[q];
         }
       }
-      for (; __ballot(q >= 0); ++steps) {
+      for (const int left = kLocalLinks - (r - r0); steps < left && __ballot(q >= 0); ++steps) {
         const int32_t stop = __hip_atomic_load(&s_fail, __ATOMIC_RELAXED, WG);   // arrives with the operands
         tx = ty = tz = false;
         if (q >= 0) {
@@ -362,13 +384,15 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
         }
       }
       nt += tight;
+      if (__ballot(q >= 0) && lane == 0) s_out = 1;  // (or it failed)
       if (lane == 0) __hip_atomic_fetch_max(&s_steps, steps, __ATOMIC_RELAXED, WG);
       const bool wave_changed = __ballot(tight != 0) != 0;
       __syncthreads();                               // every wave is done
       r += s_steps;                                  // steps count as rounds
       if (wave_changed && lane == 0) s_chg = r;
       if (s_fail) { failed_at = r; break; }
-      if (!s_over[cur]) break;                       // no marks left anywhere: the fixpoint
+      unsettled = s_out != 0;
+      if (unsettled || !s_over[cur]) break;          // no marks left anywhere: the fixpoint
       // Marks that found a stack full: a dense round (of the parity r has now).
       __syncthreads();                               // every wave has read the flags
       if (tid == 0) {
@@ -381,10 +405,10 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       __syncthreads();
     }
     // ---- results
-    const int sums[3] = {wave_sum(nt0), wave_sum(nt), wave_sum(ne)};
+    const long long sums[3] = {wave_sum64(nt0), wave_sum64(nt), wave_sum64(ne)};
     if (lane == 0)
       for (int i = 0; i < 3; ++i)
-        if (sums[i]) __hip_atomic_fetch_add(&s_sum[i], sums[i], __ATOMIC_RELAXED, WG);
+        if (sums[i]) __hip_atomic_fetch_add(&s_sum[i], (unsigned long long)sums[i], __ATOMIC_RELAXED, WG);
     if (soa) {
       for (int32_t v = tid; v < V && !start_failed; v += B) {
         const int2 b = st[v];
@@ -397,17 +421,18 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
     __syncthreads();                                 // the sums and s_chg are in
     if (tid == 0) {
       const int32_t last = s_chg - 1;                // the last round that tightened something
-      if (soa) *f = InstFlags{{-2, -1}, failed_at, r, s_sum[2], 0, -1, {-1, -1}};
+      if (soa && !job.resume) *f = InstFlags{{-2, -1}, failed_at, r, 0, 0, -1, {-1, -1}};
       if (last >= 0) f->changed[last & 1] = last;
-      if (!soa && !start_failed) {
+      if (!start_failed) {
         f->failed_at = failed_at;
         f->done_at = r;
-        f->marked_evals = s_sum[2];
+        f->marked_evals += (int64_t)s_sum[2];
+        f->settled_at = unsettled ? -1 : r;
       }
       if (job.tight) {
         const int at = slot & (kTightSlots - 1);
-        if (s_sum[0]) atomicAdd(&job.tight[at], (unsigned long long)s_sum[0]);
-        if (s_sum[1]) atomicAdd(&job.tight[kTightSlots + at], (unsigned long long)s_sum[1]);
+        if (s_sum[0]) atomicAdd(&job.tight[at], s_sum[0]);
+        if (s_sum[1]) atomicAdd(&job.tight[kTightSlots + at], s_sum[1]);
       }
     }
     if (!job.queue) return;

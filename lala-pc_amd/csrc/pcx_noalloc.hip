@@ -102,9 +102,13 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   // launch on the caller's arrays, the flags read back after it.
   if (pcx_internal::single_local(e, nvars) && e->d_adj_rec && e->adj_rec_version == e->version) {
     InstFlags f{};
-    PCX_HIP(pcx_internal::launch_single(e, d_lb, d_ub, nvars, d_flags));
-    PCX_HIP(hipMemcpyAsync(&f, d_flags, sizeof(f), hipMemcpyDeviceToHost, s));
-    PCX_HIP(hipStreamSynchronize(s));
+    bool resume = false;
+    do {
+      PCX_HIP(pcx_internal::launch_single(e, d_lb, d_ub, nvars, d_flags, resume));
+      PCX_HIP(hipMemcpyAsync(&f, d_flags, sizeof(f), hipMemcpyDeviceToHost, s));
+      PCX_HIP(hipStreamSynchronize(s));
+      resume = true;
+    } while (local_unsettled(f));
     if (out) *out = pcx_internal::single_result(e, f);
     return PCX_OK;
   }

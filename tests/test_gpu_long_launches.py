@@ -85,3 +85,64 @@ def test_a_chase_leaves_a_failed_store(gpu):
     l, u = lb.copy(), ub.copy()
     r = pir.fixpoint(l, u)
     assert r.failed and l[1] < 1000
+
+
+@pytest.mark.parametrize("c,top", [(200, 1 << 30), (20000, 1 << 30), (20000, 19000)])
+def test_a_single_store_in_lds_takes_several_launches(gpu, c, top):
+    """The LDS kernel on one store, in host memory and in the caller's device arrays;
+    counts go on from launch to launch (a step raises y by one at most)."""
+    tell, lb, ub = _climb(c, top)
+    pir = _told(tell, lb, ub)
+    l, u = lb.copy(), ub.copy()
+    r = pir.fixpoint(l, u)
+    _same(pir, r, l, u, lb, ub)
+    assert r.sweeps >= min(c, top) and r.evals >= 3 * (min(c, top) - 1)
+    d_lb, d_ub = DeviceArray(lb), DeviceArray(ub)
+    rn = pir.fixpoint_noalloc(d_lb.ptr, d_ub.ptr, len(lb))
+    _same(pir, rn, d_lb.read(), d_ub.read(), lb, ub)
+    assert rn.sweeps >= min(c, top) and rn.evals >= 3 * (min(c, top) - 1)
+    d_lb.close()
+    d_ub.close()
+
+
+@pytest.mark.parametrize("n_inst,mode", [(1, pcx.MODE_PLAIN), (1, pcx.MODE_BATCHED), (5, pcx.MODE_BATCHED),
+                                         (5, pcx.MODE_PERSISTENT), (700, pcx.MODE_BATCHED),
+                                         (700, pcx.MODE_PERSISTENT)])
+def test_batches_in_lds_take_several_launches(gpu, n_inst, mode):
+    """Instances that are done in the first launch (at their fixpoint, failed, empty
+    as loaded) beside some that need four and one that fails in its third: each
+    settled one keeps its store and its counts."""
+    tell, lb, ub = _climb(12000)
+    V = len(lb)
+    pir = _told(tell, lb, ub, base_seed=0)
+    lo, hi = np.tile(lb, (n_inst, 1)), np.tile(ub, (n_inst, 1))
+    for k in range(1, n_inst):
+        kind = k % 5
+        if kind == 1:
+            lo[k, 3] = hi[k, 3] = 50 + k                  # settles early
+        elif kind == 2:
+            hi[k, 1] = 8000                               # fails late
+        elif kind == 3:
+            lo[k, 4], hi[k, 4] = 3, 2                     # empty
+        elif kind == 4:
+            hi[k, 1] = 20                                 # fails early
+    lo_o, hi_o = lo.reshape(-1).copy(), hi.reshape(-1).copy()
+    ro = ol.fixpoint_batch(*pir.table(), lo_o, hi_o, V, threads=8)
+    b = pcx.Batch(pir, n_inst, V)
+    b.load(lo.reshape(-1), hi.reshape(-1))
+    rg, st = b.run(mode)
+    lg, ug = b.read()
+    fo = np.array([r.failed for r in ro], bool)
+    assert np.array_equal(rg.failed != 0, fo)
+    assert np.array_equal(lg.reshape(n_inst, V)[~fo], lo_o.reshape(n_inst, V)[~fo])
+    assert np.array_equal(ug.reshape(n_inst, V)[~fo], hi_o.reshape(n_inst, V)[~fo])
+    assert rg.sweeps[0] >= 12000 and rg.evals[0] >= 3 * 11999 and rg.has_changed[0]
+    assert st.full_launches >= 3                          # 12,000 steps of at most 4,096
+    for k in range(1, n_inst):
+        if k % 5 == 1:
+            assert 50 + k <= rg.sweeps[k] and rg.evals[k] < 12000
+        elif k % 5 == 3:
+            assert rg.sweeps[k] == 0 and rg.evals[k] == 0
+    b.reset()
+    lr, ur = b.read()
+    assert np.array_equal(lr, lo.reshape(-1)) and np.array_equal(ur, hi.reshape(-1))

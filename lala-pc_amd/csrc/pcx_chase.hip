@@ -18,7 +18,9 @@
 // For the same reason a wave may stop: after kChaseLinks links of a launch it drops
 // what it was chasing and only evaluates the rest of its propagators once, so that
 // a launch ends (after about 10 ms of links) however slowly the store converges,
-// and a store that another wave has failed is left within kChaseLook links.
+// and a store that another wave has failed is left within kChaseLook links.  The
+// walk of an adjacency ends when the ring is full, and a variable named by many
+// propagators (hub_degree: an objective, a makespan) is not walked at all.
 //
 // What bounds it: three dependent trips to memory a link (operands; meets;
 // adjacency records; about 2.3 us together), and the longest chain of links.  It
@@ -43,13 +45,18 @@ constexpr int kChaseVars = kWave / kChaseLanes;
 constexpr int kChaseLinks = 4096;       // links a wave chases in one launch
 constexpr int kChaseLook = 16;          // links between two looks at the store's failure (a power of two)
 
+// The adjacency a wave walks at most: eight lanes take about 0.05 us an entry, and
+// what is not walked costs a sweep of the table (5 us, and 0.03 for 1,000
+// propagators).
+int32_t hub_degree(int64_t n_props) { return (int32_t)(128 + n_props / 4096); }
+
 }  // namespace
 
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_sweep_chase(Table t, int2* st, int32_t s, InstFlags* f,
                                                         unsigned long long* tight,
                                                         const int32_t* __restrict__ adj_off,
-                                                        const int4* __restrict__ adj) {
+                                                        const int4* __restrict__ adj, int32_t hub) {
   constexpr int AG = __HIP_MEMORY_SCOPE_AGENT;
   // Sweep s runs only if sweep s-1 tightened something and nothing failed.
   if (f->changed[(s - 1) & 1] != s - 1 || f->failed_at != kNoFail) return;
@@ -127,10 +134,12 @@ __global__ __launch_bounds__(kBlock) void k_sweep_chase(Table t, int2* st, int32
       if (ty) walk[cx + below(my)] = ay;
       if (tz) walk[cy + below(mz)] = az;
       on = false;
-      for (int i0 = 0; i0 < nv; i0 += kChaseVars) {
+      for (int i0 = 0; i0 < nv && tail - head < kChaseRing; i0 += kChaseVars) {
         const int i = i0 + lane / kChaseLanes;
-        const int2 range = i < nv ? walk[i] : make_int2(0, 0);
-        for (int32_t a = range.x + (lane & (kChaseLanes - 1)); __ballot(a < range.y); a += kChaseLanes) {
+        int2 range = i < nv ? walk[i] : make_int2(0, 0);
+        if (range.y - range.x > hub) range.y = range.x;
+        for (int32_t a = range.x + (lane & (kChaseLanes - 1)); __ballot(a < range.y) && tail - head < kChaseRing;
+             a += kChaseLanes) {
           const bool got = a < range.y;
           int4 rec = make_int4(0, 0, 0, 0);
           if (got) rec = adj[a];
@@ -178,9 +187,10 @@ hipError_t launch_sweep_chase(const Table& t, int2* store, int32_t sweep, InstFl
                               hipStream_t stream) {
   if (t.n <= 0) return hipSuccess;
   const unsigned grid = (unsigned)std::min<int64_t>((t.n + kBlock - 1) / kBlock, (int64_t)cus * 4);
+  const int32_t hub = hub_degree(t.n);
   switch (dom) {
-    case kItv: k_sweep_chase<kItv><<<grid, kBlock, 0, stream>>>(t, store, sweep, flags, tight, adj_off, adj); break;
-    case kItvDiv: k_sweep_chase<kItvDiv><<<grid, kBlock, 0, stream>>>(t, store, sweep, flags, tight, adj_off, adj); break;
+    case kItv: k_sweep_chase<kItv><<<grid, kBlock, 0, stream>>>(t, store, sweep, flags, tight, adj_off, adj, hub); break;
+    case kItvDiv: k_sweep_chase<kItvDiv><<<grid, kBlock, 0, stream>>>(t, store, sweep, flags, tight, adj_off, adj, hub); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -806,7 +806,7 @@ pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
     for (; !done;) {
       // Full sweeps are timed one by one; consecutive marked sweeps as one span.
       int n_marked = 0;
-      const int count = b->chase ? (s == 0 ? pcx_internal::kChaseAfter + 2 : 2) : group;
+      const int count = b->chase ? pcx_internal::chase_count(s, group) : group;
       for (int g = 0; g < count; ++g, ++s) {
         if (e->cfg.max_sweeps > 0 && s >= e->cfg.max_sweeps) break;
         const bool marked = b->events && (s > 0 || b->seeded_run);

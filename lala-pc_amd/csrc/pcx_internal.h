@@ -154,6 +154,13 @@ hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t 
                          bool resume);
 bool chase_wanted(const pcx_engine* e);       // plain runs of one store chase
 constexpr int kChaseAfter = 4;                // plain sweeps before the first chase (see pcx_chase.hip)
+// Sweeps queued at sweep s of a run that chases before the host looks: mostly the
+// first chase finds the fixpoint and the second is quiet; a run that takes more
+// (variables too widely named to be chased) is looked at as rarely as other runs.
+inline int chase_count(int32_t s, int group) {
+  if (s == 0) return kChaseAfter + 2;
+  return s < kChaseAfter + 8 ? 2 : group;
+}
 pcx_result single_result(const pcx_engine* e, const pcx::InstFlags& f);
 }  // namespace pcx_internal
 

@@ -137,7 +137,7 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   InstFlags hf{};
   int32_t sw = 0;
   for (;;) {
-    const int count = chase ? (sw == 0 ? pcx_internal::kChaseAfter + 2 : 2) : group;
+    const int count = chase ? pcx_internal::chase_count(sw, group) : group;
     for (int g = 0; g < count; ++g, ++sw) {
       if (maxs > 0 && sw >= maxs) break;
       if (chase && sw >= pcx_internal::kChaseAfter)

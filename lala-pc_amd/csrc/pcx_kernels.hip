@@ -262,8 +262,8 @@ __device__ __forceinline__ void flush_marks(const Marker& mk) {
   if (threadIdx.x == 0) { *mk.list_n = 0; *mk.overflow = 0; }   // ordered by the caller's barrier
 }
 
-// Apply one propagator to operands already loaded.
-template <int D, int SCOPE>
+// Apply one propagator to operands already loaded (SORTED: see deduce_sorted).
+template <int D, int SCOPE, bool SORTED = false>
 __device__ __forceinline__ void apply(int2* __restrict__ st, int op, int32_t x, int32_t y,
                                       int32_t z, u64 wx, u64 wy, u64 wz, bool& chg, bool& fail,
                                       int& nt, const Marker& mk) {
@@ -280,7 +280,8 @@ __device__ __forceinline__ void apply(int2* __restrict__ st, int op, int32_t x, 
     const int2 X = as_itv(wx), Y = as_itv(wy), Z = as_itv(wz);
     if (X.x > X.y || Y.x > Y.y || Z.x > Z.y) { fail = true; return; }
     int2 nx, ny, nz;
-    deduce<D == kItvDiv>(op, X, Y, Z, nx, ny, nz);
+    if constexpr (SORTED) deduce_sorted<D == kItvDiv>(op, X, Y, Z, nx, ny, nz);
+    else deduce<D == kItvDiv>(op, X, Y, Z, nx, ny, nz);
     if (nx.x > nx.y || ny.x > ny.y || nz.x > nz.y) fail = true;
     tx = meet_itv<SCOPE>(st, x, X, nx, chg, fail, nt);
     ty = meet_itv<SCOPE>(st, y, Y, ny, chg, fail, nt);
@@ -2374,8 +2375,8 @@ __global__ __launch_bounds__(kPBlock) void k_persistent(Table t, int2* __restric
           u64 a2 = 0, b2 = 0, c2 = 0;
           if (i2 >= 0) { a2 = load_word<WG>(st + x2); b2 = load_word<WG>(st + y2); c2 = load_word<WG>(st + z2); }
           const Marker none{};
-          apply<D, WG>(st, (int)(xo1 >> kOpShift), x1, y1, z1, a1, b1, c1, chg, fail, nt, none);
-          if (i2 >= 0) apply<D, WG>(st, (int)(xo2 >> kOpShift), x2, y2, z2, a2, b2, c2, chg, fail, nt, none);
+          apply<D, WG, true>(st, (int)(xo1 >> kOpShift), x1, y1, z1, a1, b1, c1, chg, fail, nt, none);
+          if (i2 >= 0) apply<D, WG, true>(st, (int)(xo2 >> kOpShift), x2, y2, z2, a2, b2, c2, chg, fail, nt, none);
         }
         const bool wc = __ballot(chg) != 0, wf = __ballot(fail) != 0;
         if (lane == 0 && wc) s_chg = 1;

@@ -170,6 +170,7 @@ pcx_result single_result(const pcx_engine* e, const InstFlags& f) {
   r.has_changed = last >= 0;
   r.sweeps = r.failed ? (int64_t)f.failed_at + 1 : (int64_t)last + 2;
   r.evals = f.failed_at == -1 ? 0 : (int64_t)e->op.size() + f.marked_evals;
+  if (local_unsettled(f)) r.sweeps = f.done_at;
   return r;
 }
 
@@ -576,6 +577,7 @@ pcx_status plan_seed(pcx_batch* b, SeedPlan* plan) {
 constexpr int64_t kLocalBatchProps = (int64_t)1 << 17;
 bool local_wanted(const pcx_batch* b, int32_t mode, bool seeded) {
   const pcx_config& c = b->e->cfg;
+  if (b->no_local) return false;
   if (mode == PCX_MODE_PLAIN) return b->n_inst == 1 && b->h_off.empty() && !b->seeded &&
                                      pcx_internal::single_local(b->e, b->nvars);
   if (c.lds_mode == 0 || c.max_sweeps > 0 || c.event_driven == 0 || 3 * b->table_n >= ((int64_t)1 << 31) ||
@@ -601,6 +603,21 @@ pcx_status write_absent_image(pcx_batch* b) {
     PCX_HIP(launch_copy_words(b->d_store, b->d_image, b->n_inst * b->nvars, b->e->stream));
   b->image_absent = false;
   return PCX_OK;
+}
+
+// The tables and marks that sweeps of the batch read; in plain mode, adjacency
+// records instead where one store's full sweeps chase (no marks are kept then).
+pcx_status prepare_sweeps(pcx_batch* b, int32_t mode) {
+  b->chase = false;
+  const pcx_status st = prepare_tables(b);
+  return st == PCX_OK ? prepare_events(b, mode) : st;
+}
+pcx_status prepare_plain(pcx_batch* b) {
+  pcx_engine* e = b->e;
+  b->chase = !b->seeded && b->n_inst == 1 && b->h_off.empty() && pcx_internal::chase_wanted(e);
+  if (!b->chase) return prepare_sweeps(b, PCX_MODE_PLAIN);
+  b->events = b->seeded_run = false;
+  return ensure_adj_records(e);
 }
 
 pcx_status prepare_run(pcx_batch* b, int32_t mode, SeedPlan* plan, bool* local) {
@@ -643,21 +660,34 @@ pcx_status prepare_run(pcx_batch* b, int32_t mode, SeedPlan* plan, bool* local) 
     st = ensure_adj_records(e);
     return st == PCX_OK ? ensure_members(b) : st;
   }
-  b->chase = mode == PCX_MODE_PLAIN && !b->seeded && b->n_inst == 1 && b->h_off.empty() &&
-             pcx_internal::chase_wanted(e);
-  if (b->chase) {                           // full sweeps that chase: no marks are kept
-    b->events = b->seeded_run = false;
-    return ensure_adj_records(e);
-  }
-  st = prepare_tables(b);
-  if (st != PCX_OK) return st;
-  return prepare_events(b, mode);
+  return mode == PCX_MODE_PLAIN ? prepare_plain(b) : prepare_sweeps(b, mode);
+}
+
+// Persistent sweeps over the batch's stores, in LDS or in place: one launch,
+// workgroups pull whole instances from a queue ordered largest first.
+pcx_status launch_whole(pcx_batch* b, int32_t maxs, bool resume) {
+  pcx_engine* e = b->e;
+  // LDS-resident stores whenever the store fits in a workgroup's LDS (lds_mode
+  // 1 or -1): even at 128 KB, one workgroup per CU, the LDS sweep was 2.3x
+  // faster than the same sweep on global memory.
+  const int64_t sbytes = b->nvars * 8;
+  const int64_t lds_cap = lds_store_cap(e->cfg.device);
+  const bool lds = e->cfg.lds_mode != 0 && sbytes <= lds_cap;
+  const int per_cu = persistent_blocks_per_cu(dom_of(e), lds ? sbytes : 0);
+  const int grid = (int)std::min<int64_t>((int64_t)pcx_internal::device_cus(e->cfg.device) * per_cu, b->n_inst);
+  PCX_HIP(launch_persistent(run_table(b), b->d_store, b->nvars, run_subsets(b), b->table_n, b->d_flags, b->d_order,
+                            (int32_t)b->n_inst, b->d_ctl + 3, b->d_tight, maxs, dom_of(e), grid, lds, lds_cap,
+                            e->stream, resume));
+  return PCX_OK;
 }
 
 // The LDS kernel over the batch: one launch, one workgroup per instance, and
-// further ones while it left instances unsettled.
-pcx_status run_local(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
+// further ones while it left instances unsettled (sweeps once it left one for
+// them; in plain mode, *left set, the caller's, with the whole device).
+constexpr int32_t kWholeSweeps = 4096;      // sweeps of an instance in one of those launches
+pcx_status run_local(pcx_batch* b, int32_t mode, pcx_result* results, pcx_stats* stats, bool* left) {
   pcx_engine* e = b->e;
+  *left = false;
   SweepTimer tm{b, e->cfg.timing != 0};
   LocalJob job{};
   job.store = b->d_store;
@@ -677,14 +707,29 @@ pcx_status run_local(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
   for (;;) {
     pcx_status ts = tm.begin(e->stream);
     if (ts != PCX_OK) return ts;
-    PCX_HIP(launch_local(table_of(e), job, dom_of(e), e->cfg.device,
-                         pcx_internal::device_cus(e->cfg.device), e->stream));
+    if (*left) {
+      ts = launch_whole(b, kWholeSweeps, true);
+      if (ts != PCX_OK) return ts;
+    } else {
+      PCX_HIP(launch_local(table_of(e), job, dom_of(e), e->cfg.device,
+                           pcx_internal::device_cus(e->cfg.device), e->stream));
+    }
     ts = tm.end(e->stream, true);
     if (ts != PCX_OK) return ts;
     b->load_ms = load_ms;
     ts = collect(b, flags, results, stats, tm);
-    if (ts != PCX_OK || std::none_of(flags.begin(), flags.end(), local_unsettled)) return ts;
+    if (ts != PCX_OK || std::none_of(flags.begin(), flags.end(), local_unsettled)) {
+      *left = false;
+      return ts;
+    }
     job.resume = true;
+    if (!*left && std::any_of(flags.begin(), flags.end(), local_left)) {
+      *left = true;
+      b->load_ms = load_ms;
+      if (mode == PCX_MODE_PLAIN) return PCX_OK;
+      ts = prepare_tables(b);
+      if (ts != PCX_OK) return ts;
+    }
     PCX_HIP(hipMemsetAsync(job.queue, 0, sizeof(int32_t), e->stream));
   }
 }
@@ -712,8 +757,9 @@ pcx_status ensure_queue(pcx_batch* b) {
 }
 
 // Plain mode: every instance on its own, one launch per sweep, host checks
-// the instance's flags every `group` sweeps.
-pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
+// the instance's flags every `group` sweeps.  first > 0: a batch of one goes on at
+// that sweep, after the one that its flags say tightened something.
+pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats, int32_t first = 0) {
   pcx_engine* e = b->e;
   const int group = e->cfg.sweeps_per_check > 0 ? e->cfg.sweeps_per_check : 8;
   const Table t = table_of(e);
@@ -776,7 +822,7 @@ pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
     }
     int2* st = b->d_store + k * b->nvars;
     InstFlags* f = b->d_flags + k;
-    int32_t s = 0;
+    int32_t s = first;
     bool done = false;
     if (qmode && (maxs <= 0 || maxs > 1)) {
       pcx_status ts = tm.begin(e->stream);
@@ -1116,28 +1162,46 @@ pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, 
   return collect(b, flags, results, stats, tm);
 }
 
-// Persistent mode: one launch; workgroups pull whole instances from a queue
-// ordered largest first and run each to its fixpoint.
+// One store in plain mode that fits the LDS kernel, which may leave it to sweeps by
+// the whole device.
+pcx_status run_local_then_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
+  pcx_engine* e = b->e;
+  bool left = false;
+  pcx_stats ls{};
+  pcx_status s = run_local(b, PCX_MODE_PLAIN, results, &ls, &left);
+  if (stats) *stats = ls;
+  if (s != PCX_OK || !left) return s;
+  InstFlags f;
+  s = read_small(b, b->d_flags, sizeof(f), &f);
+  if (s == PCX_OK) s = prepare_plain(b);
+  if (s != PCX_OK) return s;
+  pcx_result r{};
+  pcx_stats ps{};
+  s = run_plain(b, &r, &ps, f.done_at);
+  if (s != PCX_OK) return s;
+  // run_plain counted the rounds so far as sweeps of the whole table; the first was
+  r.evals -= (int64_t)(f.done_at - 1) * b->table_n;
+  if (results) results[0] = r;
+  if (stats) {
+    ps.kernel_ms += ls.kernel_ms;
+    ps.kernel_launches += ls.kernel_launches;
+    ps.full_ms += ls.full_ms;
+    ps.full_launches += ls.full_launches;
+    ps.evals = ps.full_evals = r.evals;
+    *stats = ps;
+  }
+  return PCX_OK;
+}
+
+// Persistent mode: one launch, every instance to its fixpoint.
 pcx_status run_persistent(pcx_batch* b, pcx_result* results, pcx_stats* stats) {
   pcx_engine* e = b->e;
-  const Table t = run_table(b);
-  const int dev_cus = pcx_internal::device_cus(e->cfg.device);
-  // LDS-resident stores whenever the store fits in a workgroup's LDS (lds_mode
-  // 1 or -1): even at 128 KB, one workgroup per CU, the LDS sweep was 2.3x
-  // faster than the same sweep on global memory.
-  const int64_t sbytes = b->nvars * 8;
-  const int64_t lds_cap = lds_store_cap(e->cfg.device);
-  const bool lds = e->cfg.lds_mode != 0 && sbytes <= lds_cap;
-  const int per_cu = persistent_blocks_per_cu(dom_of(e), lds ? sbytes : 0);
-  const int grid = (int)std::min<int64_t>((int64_t)dev_cus * per_cu, b->n_inst);
-  const Subsets sub = run_subsets(b);
   const int32_t maxs = (int32_t)std::min<int64_t>(e->cfg.max_sweeps, 1 << 30);
   SweepTimer tm{b, e->cfg.timing != 0};
   pcx_status ts = tm.begin(e->stream);
   if (ts != PCX_OK) return ts;
-  PCX_HIP(launch_persistent(t, b->d_store, b->nvars, sub, b->table_n, b->d_flags, b->d_order,
-                            (int32_t)b->n_inst, b->d_ctl + 3, b->d_tight, maxs, dom_of(e), grid,
-                            lds, lds_cap, e->stream));
+  ts = launch_whole(b, maxs, false);
+  if (ts != PCX_OK) return ts;
   ts = tm.end(e->stream, true);
   if (ts != PCX_OK) return ts;
   PCX_HIP(hipStreamSynchronize(e->stream));
@@ -1707,7 +1771,7 @@ pcx_status pcx_batch_run(pcx_batch* b, int32_t mode, pcx_result* results, pcx_st
   PCX_HIP(hipSetDevice(e->cfg.device));
   const double t0 = now_ms();
   SeedPlan plan;
-  bool local = false;
+  bool local = false, left = false;
   const bool was_image = b->store_is_image;
   pcx_status s = prepare_run(b, mode, &plan, &local);
   if (s != PCX_OK) {
@@ -1715,9 +1779,9 @@ pcx_status pcx_batch_run(pcx_batch* b, int32_t mode, pcx_result* results, pcx_st
     return s;
   }
   switch (mode) {
-    case PCX_MODE_PLAIN: s = local ? run_local(b, results, stats) : run_plain(b, results, stats); break;
-    case PCX_MODE_BATCHED: s = local ? run_local(b, results, stats) : run_batched(b, plan, results, stats); break;
-    case PCX_MODE_PERSISTENT: s = local ? run_local(b, results, stats) : run_persistent(b, results, stats); break;
+    case PCX_MODE_PLAIN: s = local ? run_local_then_plain(b, results, stats) : run_plain(b, results, stats); break;
+    case PCX_MODE_BATCHED: s = local ? run_local(b, mode, results, stats, &left) : run_batched(b, plan, results, stats); break;
+    case PCX_MODE_PERSISTENT: s = local ? run_local(b, mode, results, stats, &left) : run_persistent(b, results, stats); break;
     default: return fail_with(PCX_EINVAL, "unknown mode");
   }
   if (stats) stats->wall_ms = now_ms() - t0;
@@ -2060,8 +2124,9 @@ pcx_status pcx_batch_autotune(pcx_batch* b, int32_t reps, pcx_tuning* best, pcx_
 namespace {
 // A small store through the LDS kernel: the kernel reads and writes the bounds
 // in pinned host memory itself (at most 2 x 160 KB), so a call is two host
-// copies, one launch and one wait.
-pcx_status fixpoint_local(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx_result* out) {
+// copies, one launch and one wait.  *left: the kernel left the store to sweeps, as
+// far as it came.
+pcx_status fixpoint_local(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx_result* out, bool* left) {
   PCX_HIP(hipSetDevice(e->cfg.device));
   pcx_status s = sync_table(e);
   if (s == PCX_OK) s = ensure_adj_records(e);
@@ -2083,10 +2148,11 @@ pcx_status fixpoint_local(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars
     PCX_HIP(pcx_internal::launch_single(e, plb, pub, nvars, flags, resume));
     PCX_HIP(hipStreamSynchronize(e->stream));
     resume = true;
-  } while (local_unsettled(*flags));
+  } while (local_unsettled(*flags) && !local_left(*flags));
+  *left = local_left(*flags);
   std::memcpy(lb, plb, nvars * sizeof(int32_t));
   std::memcpy(ub, pub, nvars * sizeof(int32_t));
-  if (out) *out = pcx_internal::single_result(e, *flags);
+  *out = pcx_internal::single_result(e, *flags);
   return PCX_OK;
 }
 }  // namespace
@@ -2096,7 +2162,13 @@ pcx_status pcx_fixpoint(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, 
   if (e->cfg.domain != PCX_DOMAIN_INTERVAL) return fail_with(PCX_EINVAL, "pcx_fixpoint needs an interval engine");
   if (nvars <= 0) return fail_with(PCX_EINVAL, "nvars must be positive");
   if (e->max_var >= nvars) return fail_with(PCX_EINVAL, "a propagator names a variable outside the store");
-  if (pcx_internal::single_local(e, nvars)) return fixpoint_local(e, lb, ub, nvars, out);
+  pcx_result head{};                       // what the LDS kernel did before it left the store
+  bool left = false;
+  if (pcx_internal::single_local(e, nvars)) {
+    const pcx_status s = fixpoint_local(e, lb, ub, nvars, &head, &left);
+    if (s == PCX_OK && !left && out) *out = head;
+    if (s != PCX_OK || !left) return s;
+  }
   if (!e->scratch || e->scratch_nvars != nvars || e->scratch_table != (int64_t)e->op.size()) {
     if (e->scratch) pcx_batch_destroy(e->scratch);
     e->scratch = nullptr;
@@ -2108,10 +2180,15 @@ pcx_status pcx_fixpoint(pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, 
   pcx_status s = pcx_batch_load(e->scratch, lb, ub);
   if (s != PCX_OK) return s;
   pcx_result r{};
+  e->scratch->no_local = left;
   s = pcx_batch_run(e->scratch, PCX_MODE_PLAIN, &r, nullptr);
+  e->scratch->no_local = false;
   if (s != PCX_OK) return s;
   s = pcx_batch_read(e->scratch, lb, ub);
   if (s != PCX_OK) return s;
+  r.has_changed |= head.has_changed;
+  r.sweeps += head.sweeps;
+  r.evals += head.evals;
   if (out) *out = r;
   return PCX_OK;
 }

@@ -73,6 +73,7 @@ struct pcx_batch {
   bool seeded = false;                // the next run may start from seeded marks
   bool seeded_run = false;            // this run starts with a marked sweep
   bool chase = false;                 // this run's sweeps chase what they tighten
+  bool no_local = false;              // the LDS kernel has left this store to sweeps
   bool marks_clean = false;           // both mark planes and the summaries are zero
   // first sweeps seeded from a base store (per variable the value instances
   // 0-2 agree on): the base, the values of the image that differ from it

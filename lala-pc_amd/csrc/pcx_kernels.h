@@ -309,11 +309,14 @@ constexpr int kMarkedWordsPerItem = kChunkWords;   // bitmap words per marked-sw
 constexpr int64_t kLdsStoreBytes = 64 * 1024;
 constexpr int64_t kLdsStaticReserve = 256;
 int64_t lds_store_cap(int device);
+// resume: only instances that a launch of launch_local left unsettled, from sweep
+// done_at on, max_sweeps of them (evaluations into marked_evals, settled_at set
+// where one was quiet).
 hipError_t launch_persistent(const Table& t, int2* store, int64_t nvars, const Subsets& sub,
                              int64_t n_props, InstFlags* flags, const int32_t* order,
                              int32_t n_inst, int32_t* queue, unsigned long long* tight,
                              int32_t max_sweeps, int dom, int grid, bool lds, int64_t lds_cap,
-                             hipStream_t st);
+                             hipStream_t st, bool resume = false);
 // Full sweep of one interval store whose waves chase what they tighten in the
 // same launch (pcx_chase.hip); adj: the adjacency records, adj_off their ranges.
 hipError_t launch_sweep_chase(const Table& t, int2* store, int32_t sweep, InstFlags* flags,
@@ -327,7 +330,9 @@ hipError_t launch_sweep_chase(const Table& t, int2* store, int32_t sweep, InstFl
 // the kernel reads and writes in place: memory the device can address,
 // emptiness found by the kernel, flags written whole).
 // A launch is bounded: instances that it leaves without a failure and unsettled
-// (local_unsettled) need another launch with resume set.
+// (local_unsettled) need another launch with resume set; those among them that
+// settled_at says were left for good (kLocalLeft) are better served by sweeps from
+// sweep done_at on (the sweep before it tightened something).
 struct LocalJob {
   int32_t* lb;              // or nullptr
   int32_t* ub;
@@ -344,7 +349,10 @@ struct LocalJob {
   const uint32_t* member;   // [n_inst * words], or nullptr: every propagator
   int64_t words;
   bool resume;              // go on from the stores and flags of the last launch
+  int32_t hub;              // (set by launch_local) variables of a larger degree are not walked
 };
+constexpr int32_t kLocalLeft = -2;
+inline bool local_left(const InstFlags& f) { return f.failed_at == kNoFail && f.settled_at == kLocalLeft; }
 inline bool local_unsettled(const InstFlags& f) { return f.failed_at == kNoFail && f.settled_at < 0; }
 // whether a store and a table fit (store, bitmaps and lists in LDS)
 bool local_fits(int device, int64_t nvars, int64_t n_props);

@@ -2327,7 +2327,7 @@ __global__ __launch_bounds__(kPBlock) void k_persistent(Table t, int2* __restric
                                                         InstFlags* flags, const int32_t* order,
                                                         int32_t n_inst, int32_t* queue,
                                                         unsigned long long* tight,
-                                                        int32_t max_sweeps) {
+                                                        int32_t max_sweeps, bool resume) {
   constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
   __shared__ int32_t s_slot, s_chg, s_fail;
   extern __shared__ u64 s_lds[];
@@ -2345,8 +2345,10 @@ __global__ __launch_bounds__(kPBlock) void k_persistent(Table t, int2* __restric
     const int64_t m = it.m;
     int2* gst = store + (int64_t)k * nvars;
     int2* st = LDS ? reinterpret_cast<int2*>(s_lds) : gst;
-    const bool start_failed = f->failed_at != kNoFail;
-    int32_t last_changed = -1, failed_at = kNoFail, s = 0;
+    const bool start_failed = f->failed_at != kNoFail || (resume && f->settled_at >= 0);
+    const int32_t s0 = resume ? uni(min(max(f->done_at, 0), 1 << 30)) : 0;
+    int32_t last_changed = -1, failed_at = kNoFail, s = s0;
+    bool quiet = false;
     int nt = 0;
     if (LDS && !start_failed) {
       const u64* g = reinterpret_cast<const u64*>(gst);
@@ -2354,7 +2356,7 @@ __global__ __launch_bounds__(kPBlock) void k_persistent(Table t, int2* __restric
       __syncthreads();
     }
     if (!start_failed) {
-      for (s = 0; max_sweeps <= 0 || s < max_sweeps; ++s) {
+      for (; max_sweeps <= 0 || s - s0 < max_sweeps; ++s) {
         if (threadIdx.x == 0) { s_chg = 0; s_fail = 0; }
         __syncthreads();
         bool chg = false, fail = false;
@@ -2386,7 +2388,8 @@ __global__ __launch_bounds__(kPBlock) void k_persistent(Table t, int2* __restric
         __syncthreads();                     // all read the verdict before it is reset
         if (any_chg) last_changed = s;
         if (any_fail) { failed_at = s; break; }
-        if (!any_chg) break;
+        quiet = !any_chg;
+        if (quiet) break;
       }
     }
     if (LDS && !start_failed) {
@@ -2401,6 +2404,10 @@ __global__ __launch_bounds__(kPBlock) void k_persistent(Table t, int2* __restric
       if (last_changed >= 0) f->changed[last_changed & 1] = last_changed;
       if (failed_at != kNoFail) f->failed_at = failed_at;
       f->done_at = s;
+      if (resume) {
+        f->marked_evals += (s - s0 + (quiet || failed_at != kNoFail ? 1 : 0)) * m;
+        f->settled_at = quiet ? s : -1;
+      }
     }
     __syncthreads();                         // s_slot is rewritten next round
   }
@@ -2432,7 +2439,7 @@ hipError_t launch_persistent(const Table& t, int2* store, int64_t nvars, const S
                              int64_t n_props, InstFlags* flags, const int32_t* order,
                              int32_t n_inst, int32_t* queue, unsigned long long* tight,
                              int32_t max_sweeps, int dom, int grid, bool lds, int64_t lds_cap,
-                             hipStream_t stream) {
+                             hipStream_t stream, bool resume) {
   if (lds && nvars * 8 > lds_cap) return hipErrorInvalidValue;
   const size_t sm = lds ? (size_t)nvars * 8 : 0;
   // Dynamic LDS beyond 64 KB (gfx950 has 160 KB per workgroup) is requested
@@ -2445,7 +2452,7 @@ hipError_t launch_persistent(const Table& t, int2* store, int64_t nvars, const S
       if (fe != hipSuccess) return fe;                                                         \
     }                                                                                          \
     k_persistent<D, L><<<grid, kPBlock, sm, stream>>>(t, store, nvars, sub, n_props, flags, order, \
-                                                      n_inst, queue, tight, max_sweeps);       \
+                                                      n_inst, queue, tight, max_sweeps, resume); \
   } while (0)
   switch (dom) {
     case kItv: if (lds) PCX_PERSIST(kItv, true); else PCX_PERSIST(kItv, false); break;

@@ -98,6 +98,7 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   hipStream_t s = e->stream;
   const int dom = pcx_internal::dom_of(e);
 
+  pcx_result head{};                   // what the LDS kernel did, when it leaves the store to sweeps
   // A small store whose adjacency records an earlier pcx_fixpoint built: one
   // launch on the caller's arrays, the flags read back after it.
   if (pcx_internal::single_local(e, nvars) && e->d_adj_rec && e->adj_rec_version == e->version) {
@@ -108,9 +109,12 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
       PCX_HIP(hipMemcpyAsync(&f, d_flags, sizeof(f), hipMemcpyDeviceToHost, s));
       PCX_HIP(hipStreamSynchronize(s));
       resume = true;
-    } while (local_unsettled(f));
-    if (out) *out = pcx_internal::single_result(e, f);
-    return PCX_OK;
+    } while (local_unsettled(f) && !local_left(f));
+    head = pcx_internal::single_result(e, f);
+    if (!local_left(f)) {
+      if (out) *out = head;
+      return PCX_OK;
+    }
   }
 
   // Every value the sweeps read is written first: flags, counters, store.
@@ -162,6 +166,9 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
     r.sweeps = r.failed ? (int64_t)hf.failed_at + 1 : (int64_t)last + 2;
     if (maxs > 0 && r.sweeps > maxs) r.sweeps = maxs;
     r.evals = r.sweeps * m + hf.marked_evals;    // (evaluations of chases)
+    r.has_changed |= head.has_changed;
+    r.sweeps += head.sweeps;
+    r.evals += head.evals;
     *out = r;
   }
   return PCX_OK;

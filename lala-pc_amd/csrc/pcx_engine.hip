@@ -101,30 +101,32 @@ int dom_of(const pcx_engine* e) {
 }
 
 // Variable -> table positions adjacency of the engine's table (each
-// propagator listed once per distinct variable), built on the host when the
-// table changed and uploaded.
+// propagator listed once per distinct variable), built on the device when the
+// table changed; complete on return, for readers on other streams.
 pcx_status ensure_adjacency(pcx_engine* e) {
-  if (e->d_adj_off && e->adj_version == e->version) return PCX_OK;
+  pcx_status st = sync_table(e);
+  if (st != PCX_OK || (e->d_adj_off && e->adj_version == e->version)) return st;
   const int64_t n = (int64_t)e->op.size();
   const int64_t V = (int64_t)e->max_var + 1;
-  std::vector<int32_t> off(V + 1, 0);
-  auto each = [&](int64_t i, auto&& f) {
-    const int32_t x = e->x[i], y = e->y[i], z = e->z[i];
-    f(x);
-    if (y != x) f(y);
-    if (z != x && z != y) f(z);
-  };
-  for (int64_t i = 0; i < n; ++i) each(i, [&](int32_t v) { ++off[v + 1]; });
-  for (int64_t v = 0; v < V; ++v) off[v + 1] += off[v];
-  std::vector<int32_t> adj(std::max<int32_t>(off[V], 1)), pos(off.begin(), off.end() - 1);
-  for (int64_t i = 0; i < n; ++i) each(i, [&](int32_t v) { adj[pos[v]++] = (int32_t)i; });
   dfree(e->d_adj_off); dfree(e->d_adj);
   PCX_HIP(hipMalloc(&e->d_adj_off, (V + 1) * sizeof(int32_t)));
-  PCX_HIP(hipMalloc(&e->d_adj, adj.size() * sizeof(int32_t)));
-  PCX_HIP(hipMemcpy(e->d_adj_off, off.data(), (V + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
-  PCX_HIP(hipMemcpy(e->d_adj, adj.data(), adj.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  PCX_HIP(hipMalloc(&e->d_adj, std::max<int64_t>(3 * n, 1) * sizeof(int32_t)));
+  int32_t total = 0;
+  if (n > 0) {
+    int32_t* scratch = nullptr;
+    PCX_HIP(hipMalloc(&scratch, adj_scratch(V) * sizeof(int32_t)));
+    hipError_t he = launch_adjacency(Table{e->d_xo, e->d_y, e->d_z, n}, V, e->d_adj_off, e->d_adj, scratch, e->stream);
+    if (he == hipSuccess)
+      he = hipMemcpyAsync(&total, e->d_adj_off + V, sizeof(total), hipMemcpyDeviceToHost, e->stream);
+    const hipError_t se = hipStreamSynchronize(e->stream);   // nothing queued still uses the scratch
+    (void)hipFree(scratch);
+    PCX_HIP(he);
+    PCX_HIP(se);
+  } else {
+    PCX_HIP(hipMemset(e->d_adj_off, 0, (V + 1) * sizeof(int32_t)));
+  }
   e->adj_vars = V;
-  e->adj_n = off[V];
+  e->adj_n = total;
   e->adj_version = e->version;
   return PCX_OK;
 }

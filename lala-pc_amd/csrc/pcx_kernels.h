@@ -357,6 +357,12 @@ inline bool local_unsettled(const InstFlags& f) { return f.failed_at == kNoFail 
 // whether a store and a table fit (store, bitmaps and lists in LDS)
 bool local_fits(int device, int64_t nvars, int64_t n_props);
 hipError_t launch_local(const Table& t, const LocalJob& job, int dom, int device, int cus, hipStream_t st);
+// The adjacency of a table (pcx_adj.hip) whose variables are below nvars: off
+// [nvars + 1], adj [up to 3 n] (fewer where a propagator names a variable twice);
+// scratch: adj_scratch(nvars) words.
+int64_t adj_scratch(int64_t nvars);
+hipError_t launch_adjacency(const Table& t, int64_t nvars, int32_t* off, int32_t* adj, int32_t* scratch,
+                            hipStream_t st);
 // rec[i] = {adj[i], xo, y, z of that propagator} for n adjacency entries
 hipError_t launch_adj_records(const Table& t, const int32_t* adj, int64_t n, int4* rec, hipStream_t st);
 // resident workgroups per CU (lds_bytes of dynamic LDS per workgroup)

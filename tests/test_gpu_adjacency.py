@@ -70,6 +70,8 @@ def test_lds_runs(gpu, n, V):
     tell, lb, ub = _chain(n, V, rng)
     pir = _tell(tell, lb, ub)
     _check(pir, lb, ub, _single)
+    if n + 2 == V:
+        return
     # told more: another table (every second link's variable below one that had no name)
     last = np.full(len(tell[1][::2]), V - 1, np.int32)
     pir.tell(np.full(len(last), pcx.LEQ), np.zeros(len(last), np.int32), tell[1][::2], last, lb, ub)

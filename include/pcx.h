@@ -313,18 +313,24 @@ typedef struct {
   int32_t lds_mode;         /* persistent: 0 or 1 (stores staged in LDS)        */
   int32_t compact_tables;   /* 0 or 1 (only varied for batches with subsets)    */
   int32_t stream_tables;    /* 0 or 1                                           */
-  int32_t event_driven;     /* batched: 0 or 1                                  */
+  int32_t event_driven;     /* batched: 0 or 1; persistent: 0 (full sweeps), or
+                               -1 (event-driven in LDS where a batch takes it)  */
   int32_t lockstep;         /* batched: 0, 16, 32 or 64                         */
   double  ms;               /* best host time of one reset + run; < 0: failed   */
 } pcx_tuning;
 
 /* Time every point of {batched: props_per_wave x compact x stream x
- * event_driven, and lockstep 16/32/64 with event_driven} U {persistent: lds (where the store fits) x compact} on the
- * batch's loaded image (one warm-up and `reps` timed runs per point, best
- * kept; the points shape the full sweeps and the sweeps after them, so the
- * runs take a full first sweep whatever base_seed says), set the engine's
- * configuration to the fastest point, and restore the stores to the image.  results (may be NULL): up to max_results points
- * in the order tried; *n_results (may be NULL) receives how many were tried.
+ * event_driven, and lockstep 16/32/64 with event_driven} U {persistent: full
+ * sweeps in memory x compact, in LDS (where the store fits), and as the
+ * automatic settings run it there} on the batch's loaded image (one warm-up
+ * and `reps` timed runs per point, best kept; the points shape the full sweeps
+ * and the sweeps after them, so the runs take a full first sweep whatever
+ * base_seed says), set the engine's configuration to the fastest point, and
+ * restore the stores to the image.  The point shapes batches: pcx_fixpoint and
+ * plain runs of one store go on choosing their kernel by the settings given at
+ * creation or to pcx_set_config.  results (may be NULL): up to max_results
+ * points in the order tried; *n_results (may be NULL) receives how many were
+ * tried.
  * No counterpart in the reference (its fixpoint has no tuning parameters). */
 pcx_status pcx_batch_autotune(pcx_batch* b, int32_t reps, pcx_tuning* best,
                               pcx_tuning* results, int32_t max_results,

@@ -138,7 +138,7 @@ pcx_status ensure_adjacency(pcx_engine* e) {
 // and runs to the fixpoint only.
 constexpr int64_t kLocalSingleProps = 16 * 1024;
 bool single_local(const pcx_engine* e, int64_t nvars) {
-  const pcx_config& c = e->cfg;
+  const pcx_config& c = e->given;
   const int64_t n = (int64_t)e->op.size();
   return c.domain == PCX_DOMAIN_INTERVAL && c.lds_mode != 0 && c.max_sweeps <= 0 && c.event_driven < 0 &&
          c.props_per_wave == 0 && c.mark_queue < 0 && n <= kLocalSingleProps && local_fits(c.device, nvars, n);
@@ -180,7 +180,7 @@ pcx_result single_result(const pcx_engine* e, const InstFlags& f) {
 // settings, runs to the fixpoint, and the adjacency records there or room for
 // them (a quarter of free memory).
 bool chase_wanted(const pcx_engine* e) {
-  const pcx_config& c = e->cfg;
+  const pcx_config& c = e->given;
   const int64_t n = (int64_t)e->op.size();
   if (c.domain != PCX_DOMAIN_INTERVAL || c.max_sweeps > 0 || c.event_driven >= 0 || c.props_per_wave != 0 ||
       c.mark_queue >= 0 || n == 0 || 3 * n >= ((int64_t)1 << 31))
@@ -1268,7 +1268,7 @@ pcx_status pcx_create(const pcx_config* cfg, pcx_engine** out) {
   PCX_HIP(hipSetDevice(c.device));
   auto* e = new (std::nothrow) pcx_engine();
   if (!e) return fail_with(PCX_ENOMEM, "host allocation failed");
-  e->cfg = c;
+  e->cfg = e->given = c;
   hipError_t he = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
   if (he != hipSuccess) {
     delete e;
@@ -1366,7 +1366,7 @@ pcx_status pcx_set_config(pcx_engine* e, const pcx_config* cfg) {
     return fail_with(PCX_EINVAL, "mark_queue must be -1 (auto), 0 (off) or a log2 capacity in [10, 26]");
   if (!valid_base_seed(cfg->base_seed))
     return fail_with(PCX_EINVAL, "base_seed must be -1 (auto), 0 (off) or 1 (on)");
-  e->cfg = *cfg;
+  e->cfg = e->given = *cfg;
   return PCX_OK;
 }
 
@@ -2080,10 +2080,15 @@ pcx_status pcx_batch_autotune(pcx_batch* b, int32_t reps, pcx_tuning* best, pcx_
   if (b->n_inst >= 2)
     for (int gi : {16, 32, 64})
       pts.push_back(pcx_tuning{PCX_MODE_BATCHED, 512, 0, 0, 0, 1, gi, 0.0});
+  // Persistent runs by full sweeps, and (stores in LDS) as the automatic settings
+  // choose: the event-driven kernel where it takes the batch, which reads the shared
+  // table, so that with subsets the sweeps are left to the point with their copies.
   const bool lds_fits = b->nvars * 8 <= lds_store_cap(e->cfg.device);
-  for (int l = 0; l <= (lds_fits ? 1 : 0); ++l)
-    for (int c = 0; c <= (subsets ? 1 : 0); ++c)
-      pts.push_back(pcx_tuning{PCX_MODE_PERSISTENT, 0, l, c, 0, 0, 0, 0.0});
+  for (int c = 0; c <= (subsets ? 1 : 0); ++c) pts.push_back(pcx_tuning{PCX_MODE_PERSISTENT, 0, 0, c, 0, 0, 0, 0.0});
+  if (lds_fits) {
+    pts.push_back(pcx_tuning{PCX_MODE_PERSISTENT, 0, 1, 0, 0, -1, 0, 0.0});
+    pts.push_back(pcx_tuning{PCX_MODE_PERSISTENT, 0, 1, subsets ? 1 : 0, 0, 0, 0, 0.0});
+  }
   int best_i = -1;
   for (size_t i = 0; i < pts.size(); ++i) {
     pcx_tuning& p = pts[i];

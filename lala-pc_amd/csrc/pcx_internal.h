@@ -10,6 +10,8 @@
 
 struct pcx_engine {
   pcx_config cfg{};
+  pcx_config given{};                 // as the caller set it: autotuning a batch changes cfg only, and
+                                      // single stores choose their kernel by these settings
   std::vector<int32_t> op, x, y, z;   // table in engine order
   int32_t max_var = -1;
   bool has_div = false;               // table holds a division propagator

@@ -2012,8 +2012,9 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   const int64_t n = b->n_inst;
   const Table t = table_of(e);
   const Subsets sub{b->h_off.empty() ? nullptr : b->d_off, b->d_idx};
-  // One buffer for the call's arrays, kept with the batch; the positions' too
-  // while they are few.
+  // One buffer for the call's arrays, kept with the batch; the positions' too where
+  // the caller's room for them is small.  Where it is not (a safe bound may be
+  // gigabytes) they are written once their number is known, into as much.
   int64_t most = b->h_off.empty() ? b->table_n : 0;
   for (int64_t k = 0; k < n && !b->h_off.empty(); ++k) most = std::max(most, inst_size(b, k));
   const int64_t chunks = ask_chunks(most), cells = n * chunks;
@@ -2023,7 +2024,7 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   const int64_t at_out = at_empty + up(n * sizeof(int32_t));
   const int64_t pairs = b->h_off.empty() ? n * b->table_n : b->h_off.back();
   const int64_t room = live_idx ? std::max<int64_t>(0, std::min(cap, pairs)) : 0;
-  const bool kept = room * (int64_t)sizeof(int32_t) <= kAskKeep;
+  const bool kept = room <= kAskKeep / (int64_t)sizeof(int32_t);
   st = ask_room(b, at_out + (kept ? room * sizeof(int32_t) : 0));
   if (st != PCX_OK) return st;
   AskWork w{};
@@ -2033,15 +2034,14 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   w.off = reinterpret_cast<int64_t*>(b->d_ask + at_off);
   w.empty = reinterpret_cast<int32_t*>(b->d_ask + at_empty);
   int32_t* d_big = nullptr;
-  if (!kept) PCX_HIP(hipMalloc(&d_big, room * sizeof(int32_t)));
-  int32_t* const d_out = kept ? reinterpret_cast<int32_t*>(b->d_ask + at_out) : d_big;
+  int32_t* d_out = kept ? reinterpret_cast<int32_t*>(b->d_ask + at_out) : nullptr;
   std::vector<int64_t> off(n + 1, 0);
   std::vector<int32_t> empty(n);
   hipError_t he = hipMemsetAsync(w.empty, 0, n * sizeof(int32_t), e->stream);
   if (he == hipSuccess)
     he = launch_ask_bits(t, b->d_store, b->nvars, sub, b->table_n, n, chunks, w, e->cfg.device,
                          pcx_internal::device_cus(e->cfg.device), e->stream);
-  if (he == hipSuccess) he = launch_ask_write(sub, n, chunks, w, d_out, room, e->stream);
+  if (he == hipSuccess && kept) he = launch_ask_write(sub, n, chunks, w, d_out, room, e->stream);
   if (he == hipSuccess)
     he = hipMemcpyAsync(off.data(), w.off, (n + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, e->stream);
   if (he == hipSuccess && extractable)
@@ -2049,10 +2049,17 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   const hipError_t se = hipStreamSynchronize(e->stream);
   if (he == hipSuccess) he = se;
   const bool fits = !live_idx || off[n] <= cap;
+  if (he == hipSuccess && fits && !kept && off[n] > 0) {
+    he = hipMalloc(&d_big, off[n] * sizeof(int32_t));
+    d_out = d_big;
+    if (he == hipSuccess) he = launch_ask_write(sub, n, chunks, w, d_out, off[n], e->stream);
+  }
   if (he == hipSuccess && fits && live_idx && off[n] > 0)
     he = copy_to_host(live_idx, off[n] * sizeof(int32_t), nullptr, 0, d_out, e->cfg.device, e->stream);
   if (d_big) (void)hipFree(d_big);
-  if (he != hipSuccess) return fail_with(PCX_EDEVICE, std::string("batch ask: ") + hipGetErrorString(he));
+  if (he != hipSuccess)
+    return fail_with(he == hipErrorOutOfMemory ? PCX_ENOMEM : PCX_EDEVICE,
+                     std::string("batch ask: ") + hipGetErrorString(he));
   if (extractable)
     for (int64_t k = 0; k < n; ++k) extractable[k] = !empty[k] && off[k + 1] == off[k];
   if (live_off) std::copy(off.begin(), off.end(), live_off);

@@ -1,0 +1,46 @@
+"""pcx_batch_ask where the caller's room for positions is far above their number: a
+safe bound costs neither device memory nor time, and the answers are those of a
+call with exactly enough room."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import pcx
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    if pcx.device_count() < 1:
+        pytest.fail("no HIP device visible: GPU tests need an MI355X")
+    return True
+
+
+def _sums(P, V, seed):
+    """P sums i + j = k over V variables whose solution is their own number."""
+    rng = np.random.default_rng(seed)
+    y = rng.integers(0, V // 2, P)
+    z = rng.integers(0, V // 2, P)
+    return np.full(P, pcx.ADD, np.int32), (y + z).astype(np.int32), y.astype(np.int32), z.astype(np.int32)
+
+
+# 20 M pairs: positions of all of them are above the 64 MB kept; 80,000 M pairs: above
+# the device's memory (320 GB).
+@pytest.mark.parametrize("n,V,P", [(400, 1000, 50000), (80000, 100, 1000000)])
+def test_room_for_every_pair(gpu, n, V, P):
+    pir = pcx.PIR()
+    pir.tell(*_sums(P, V, n))
+    lo = np.tile(np.arange(V, dtype=np.int32), (n, 1))
+    hi = lo.copy()
+    hi[3, 7] += 1                                        # open in two stores
+    hi[n - 1, V // 2] += 2
+    b = pcx.Batch(pir, n, V)
+    b.load(lo.reshape(-1), hi.reshape(-1))
+    ext, off, idx = b.ask()
+    assert np.array_equal(np.nonzero(~ext)[0], [3, n - 1]) and 0 < len(idx) < 10 * P
+    off2, idx2 = np.zeros(n + 1, np.int64), np.full(len(idx) + 8, -7, np.int32)
+    st = pcx.lib().pcx_batch_ask(b._h, None, pcx._p64(off2), pcx._p32(idx2), ctypes.c_int64(n * P))
+    assert st == pcx.OK, pcx.lib().pcx_last_error()
+    assert np.array_equal(off2, off) and np.array_equal(idx2[:len(idx)], idx) and (idx2[len(idx):] == -7).all()

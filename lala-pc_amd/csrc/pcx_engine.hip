@@ -1895,9 +1895,12 @@ bool trees_valid(const int32_t* nodes, int64_t n_nodes, const int64_t* off, int6
 }  // namespace
 
 namespace {
-// Room for an ask's arrays, kept with the batch (the positions of pcx_batch_ask up
-// to kAskKeep bytes).
+// Room for an ask's arrays, kept with the batch up to kAskKeep bytes, as is the
+// interleaved copy that formulas are asked on, up to kCopyKeep (sweeps may have made
+// one before, and keep it): what is larger is given back when the call ends, whose
+// work on so much outweighs the allocation.
 constexpr int64_t kAskKeep = (int64_t)64 << 20;
+constexpr int64_t kCopyKeep = (int64_t)256 << 20;
 pcx_status ask_room(pcx_batch* b, int64_t bytes) {
   if (b->ask_bytes >= bytes) return PCX_OK;
   dfree(b->d_ask);
@@ -1906,6 +1909,22 @@ pcx_status ask_room(pcx_batch* b, int64_t bytes) {
   b->ask_bytes = bytes;
   return PCX_OK;
 }
+struct AskTrim {
+  pcx_batch* b;
+  bool had_copy;
+  explicit AskTrim(pcx_batch* batch) : b(batch), had_copy(batch->d_shadow != nullptr) {}
+  ~AskTrim() {                          // (the stream is idle, or the frees wait for it)
+    if (b->ask_bytes > kAskKeep) {
+      dfree(b->d_ask);
+      b->ask_bytes = 0;
+    }
+    if (!had_copy && b->shadow_words * (int64_t)sizeof(int2) > kCopyKeep) {
+      dfree(b->d_shadow);
+      b->shadow_words = 0;
+      b->shadow_is_image = false;
+    }
+  }
+};
 
 // Stores from which on formulas are asked a wave's lanes at a time.
 constexpr int64_t kLanesMin = 16;
@@ -1946,6 +1965,7 @@ pcx_status pcx_batch_ask_formulas(pcx_batch* b, const int32_t* nodes, int64_t n_
   auto up = [](int64_t bytes) { return (bytes + 255) & ~(int64_t)255; };
   const int64_t at_off = up(n_nodes * sizeof(int4)), at_ok = at_off + up((n_formulas + 1) * sizeof(int64_t));
   const int64_t at_empty = at_ok + up(b->n_inst * sizeof(int32_t)), at_verdict = at_empty + up(b->n_inst);
+  const AskTrim trim(b);
   pcx_status ws = ask_room(b, at_verdict + 2 * sizeof(int32_t));
   if (ws != PCX_OK) return ws;
   int4* d_nodes = reinterpret_cast<int4*>(b->d_ask);
@@ -2025,6 +2045,7 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   const int64_t pairs = b->h_off.empty() ? n * b->table_n : b->h_off.back();
   const int64_t room = live_idx ? std::max<int64_t>(0, std::min(cap, pairs)) : 0;
   const bool kept = room <= kAskKeep / (int64_t)sizeof(int32_t);
+  const AskTrim trim(b);
   st = ask_room(b, at_out + (kept ? room * sizeof(int32_t) : 0));
   if (st != PCX_OK) return st;
   AskWork w{};

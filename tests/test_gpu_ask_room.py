@@ -6,7 +6,9 @@ import ctypes
 import numpy as np
 import pytest
 
+import pc_ask as pa
 import pcx
+import pcx.device
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +46,33 @@ def test_room_for_every_pair(gpu, n, V, P):
     st = pcx.lib().pcx_batch_ask(b._h, None, pcx._p64(off2), pcx._p32(idx2), ctypes.c_int64(n * P))
     assert st == pcx.OK, pcx.lib().pcx_last_error()
     assert np.array_equal(off2, off) and np.array_equal(idx2[:len(idx)], idx) and (idx2[len(idx):] == -7).all()
+
+
+def _free():
+    h = pcx.device._runtime()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert h.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_large_work_arrays_are_given_back(gpu):
+    """4,096 stores: 200 MB of answer bits at 400,000 propagators, a 640 MB copy for
+    formulas at 20,000 variables.  What a batch keeps between calls stays below 64 MB."""
+    n, V, P = 4096, 20000, 400000
+    pir = pcx.PIR()
+    pir.tell(*_sums(P, V, 1))
+    lo = np.tile(np.arange(V, dtype=np.int32), (n, 1)).reshape(-1)
+    hi = lo.copy()
+    hi[5 * V + 9] += 1
+    b = pcx.Batch(pir, n, V)
+    b.load(lo, hi)
+    b.ask(live=False)                                    # the table goes to the device
+    before = _free()
+    nodes = np.array([[pa.VAR, 9, 0, 0], [pa.CONST, 9, 0, 0], [pa.EQ, 0, 0, 0]] * 1000, np.int32)
+    for _ in range(2):
+        ext, _, idx = b.ask()
+        assert np.array_equal(np.nonzero(~ext)[0], [5]) and len(idx) > 0
+        got = b.ask_formulas(nodes, np.arange(0, 3001, 3, dtype=np.int64))
+        assert np.array_equal(np.nonzero(~got)[0], [5])
+    assert before - _free() < 96 << 20
+    assert np.array_equal(b.read()[1], hi)

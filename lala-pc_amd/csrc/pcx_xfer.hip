@@ -15,8 +15,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "pcx_xfer.h"
@@ -114,7 +114,7 @@ hipError_t share_out(size_t bytes, int device, F carry) {
   for (int t = 1; t < threads; ++t) {
     try {
       th[t] = std::thread(work, t);
-    } catch (const std::system_error&) {        // no thread to be had: the caller carries this share too
+    } catch (const std::exception&) {           // no thread or no memory for one: the caller carries this share too
       work(t);
     }
   }

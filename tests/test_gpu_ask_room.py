@@ -68,11 +68,40 @@ def test_large_work_arrays_are_given_back(gpu):
     b.load(lo, hi)
     b.ask(live=False)                                    # the table goes to the device
     before = _free()
-    nodes = np.array([[pa.VAR, 9, 0, 0], [pa.CONST, 9, 0, 0], [pa.EQ, 0, 0, 0]] * 1000, np.int32)
+    nodes = np.array([[pa.VAR, 9, 0, 0], [pa.CONST, 9, 0, 0], [pa.EQ, 0, 0, 0]] * 14000, np.int32)
     for _ in range(2):
         ext, _, idx = b.ask()
         assert np.array_equal(np.nonzero(~ext)[0], [5]) and len(idx) > 0
-        got = b.ask_formulas(nodes, np.arange(0, 3001, 3, dtype=np.int64))
+        got = b.ask_formulas(nodes, np.arange(0, 42001, 3, dtype=np.int64))
         assert np.array_equal(np.nonzero(~got)[0], [5])
     assert before - _free() < 96 << 20
     assert np.array_equal(b.read()[1], hi)
+
+
+@pytest.mark.parametrize("V", [1000, 100000])
+def test_few_formulas_copy_no_stores(gpu, V):
+    """Below two nodes a variable the stores are not interleaved for an ask (51 MB at
+    100,000 variables), and the answers are those of the lanes' kernel from there on."""
+    n = 64
+    lo = np.tile(np.arange(V, dtype=np.int32), (n, 1))
+    hi = lo.copy()
+    hi[7, 3] += 1
+    lo[9, 5], hi[9, 5] = 4, 2                             # an empty store
+    b = pcx.Batch(pcx.PIR(), n, V)
+    b.load(lo.reshape(-1), hi.reshape(-1))
+    tree = [[pa.VAR, 3, 0, 0], [pa.CONST, 3, 0, 0], [pa.EQ, 0, 0, 0]]
+    want = ~np.isin(np.arange(n), (7, 9))
+
+    def ask(m):
+        off = np.arange(m + 1, dtype=np.int64) * 3
+        return b.ask_formulas(np.array(tree * m, np.int32), off)
+
+    assert np.array_equal(ask(1), want)
+    before = _free()
+    for m in (1, 50, (2 * V - 1) // 3):                  # up to one node short of the rule
+        assert np.array_equal(ask(m), want)
+    assert before - _free() < 24 << 20
+    for m in ((2 * V + 2) // 3, V):
+        assert np.array_equal(ask(m), want)
+    lo2, hi2 = b.read()
+    assert np.array_equal(lo2, lo.reshape(-1)) and np.array_equal(hi2, hi.reshape(-1))

@@ -2070,9 +2070,16 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
   if (he == hipSuccess)
     he = launch_ask_bits(t, b->d_store, b->nvars, sub, b->table_n, n, chunks, w, e->cfg.device,
                          pcx_internal::device_cus(e->cfg.device), e->stream);
-  if (he == hipSuccess && kept) he = launch_ask_write(sub, n, chunks, w, d_out, room, e->stream);
-  if (he == hipSuccess)
-    he = hipMemcpyAsync(off.data(), w.off, (n + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, e->stream);
+  // Who asks only whether stores are extractable needs no places: the counts.
+  std::vector<int32_t> count(live_off ? 0 : cells);
+  if (live_off) {
+    if (he == hipSuccess) he = launch_ask_places(n, chunks, w, e->stream);
+    if (he == hipSuccess && kept) he = launch_ask_write(sub, n, chunks, w, d_out, room, e->stream);
+    if (he == hipSuccess)
+      he = hipMemcpyAsync(off.data(), w.off, (n + 1) * sizeof(int64_t), hipMemcpyDeviceToHost, e->stream);
+  } else if (he == hipSuccess) {
+    he = hipMemcpyAsync(count.data(), w.count, cells * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
+  }
   if (he == hipSuccess && extractable)
     he = hipMemcpyAsync(empty.data(), w.empty, n * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
   const hipError_t se = hipStreamSynchronize(e->stream);
@@ -2090,7 +2097,10 @@ pcx_status pcx_batch_ask(pcx_batch* b, int32_t* extractable, int64_t* live_off, 
     return fail_with(he == hipErrorOutOfMemory ? PCX_ENOMEM : PCX_EDEVICE,
                      std::string("batch ask: ") + hipGetErrorString(he));
   if (extractable)
-    for (int64_t k = 0; k < n; ++k) extractable[k] = !empty[k] && off[k + 1] == off[k];
+    for (int64_t k = 0; k < n; ++k)
+      extractable[k] = !empty[k] && off[k + 1] == off[k] &&
+                       (live_off || std::all_of(count.begin() + k * chunks, count.begin() + (k + 1) * chunks,
+                                                [](int32_t c) { return c == 0; }));
   if (live_off) std::copy(off.begin(), off.end(), live_off);
   if (!fits)
     return fail_with(PCX_EINVAL, "live_idx capacity too small (live_off[n_inst] holds the size needed)");

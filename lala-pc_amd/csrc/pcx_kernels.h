@@ -401,9 +401,11 @@ struct AskWork {
   int32_t* empty;           // [n_inst]: 1 where the store holds an empty interval (zeroed by the caller)
 };
 int64_t ask_chunks(int64_t most_props);
-// everything but the positions
+// bits, counts and emptiness
 hipError_t launch_ask_bits(const Table& t, const int2* store, int64_t nvars, const Subsets& sub, int64_t n_props,
                            int64_t n_inst, int64_t chunks, const AskWork& w, int device, int cus, hipStream_t st);
+// places and offsets
+hipError_t launch_ask_places(int64_t n_inst, int64_t chunks, const AskWork& w, hipStream_t st);
 // the positions, in the order of the instances, as far as cap
 hipError_t launch_ask_write(const Subsets& sub, int64_t n_inst, int64_t chunks, const AskWork& w, int32_t* out,
                             int64_t cap, hipStream_t st);

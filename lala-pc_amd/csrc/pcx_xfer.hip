@@ -8,9 +8,11 @@
 // out.  (The other direction, from arrays a program has already written, is
 // faster through the runtime: 24 MB in 0.9 ms, and 1.0 this way.)
 //
-// The slots (kThreads * 2 * kSlot bytes, allocated on the first large copy) are
-// one pool for the process, freed with the last engine.  A copy that finds the
-// pool in use by another thread takes the runtime's path.
+// The slots (kThreads * 2 * kSlot bytes) are one pool for the process, freed with the
+// last engine.  Their allocation takes 0.9 ms, which a copy of a few megabytes does not
+// win back: they are made once copies of kWorth bytes have gone the runtime's way, so
+// that a program that makes an engine, reads its results and drops it pays for none.
+// A copy that finds the pool in use by another thread takes the runtime's path.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,6 +30,7 @@ namespace {
 // 512 and 256 KB took 1.4 and 2.0.
 constexpr int kThreads = 4;
 constexpr size_t kSlot = (size_t)1 << 20;
+constexpr size_t kWorth = (size_t)32 << 20;     // what they save, about 26 us a megabyte, by then
 constexpr size_t kShare = (size_t)1 << 20;      // bytes a further thread is worth starting for
 
 struct Pool {
@@ -35,6 +38,7 @@ struct Pool {
   std::mutex life;                              // users, and the slots' life
   int users = 0;
   uint8_t* slots = nullptr;
+  size_t waited = 0;                            // bytes of large copies before there were slots
   hipEvent_t ev[2 * kThreads] = {};
   int device = -1;                              // the events' device
 };
@@ -48,8 +52,10 @@ void drop_events() {
   g_pool.device = -1;
 }
 
-// Slots and events for `device` (the current one); the caller holds `use`.
-bool ready(int device) {
+// Slots and events for `device` (the current one), if copies like this one of `bytes`
+// are worth them; the caller holds `use`.
+bool ready(int device, size_t bytes) {
+  if (!g_pool.slots && (g_pool.waited += std::min(bytes, kWorth)) <= kWorth) return false;
   if (!g_pool.slots &&
       hipHostMalloc(reinterpret_cast<void**>(&g_pool.slots), 2 * kThreads * kSlot, hipHostMallocPortable) != hipSuccess) {
     (void)hipGetLastError();
@@ -143,13 +149,14 @@ void xfer_release() {
   drop_events();
   if (g_pool.slots) (void)hipHostFree(g_pool.slots);
   g_pool.slots = nullptr;
+  g_pool.waited = 0;
 }
 
 hipError_t copy_to_host(void* dst, size_t bytes, void* dst2, size_t bytes2, const void* src, int device,
                         hipStream_t st) {
   if (bytes + bytes2 >= kXferMin) {
     std::unique_lock<std::mutex> l(g_pool.use, std::try_to_lock);
-    if (l.owns_lock() && ready(device)) {
+    if (l.owns_lock() && ready(device, bytes + bytes2)) {
       const Dest to{static_cast<uint8_t*>(dst), bytes, static_cast<uint8_t*>(dst2)};
       const hipError_t he = share_out(bytes + bytes2, device, [&](int t, size_t at, size_t end) {
         return carry_out(t, to, static_cast<const uint8_t*>(src), at, end, st);

@@ -12,9 +12,17 @@ typedef int* hipEvent_t;
 constexpr unsigned hipHostMallocPortable = 1, hipEventDisableTiming = 2;
 
 extern int g_fail_copies;                       // copies that fail from now on
+extern int g_pinned;                            // pinned allocations alive
 
-inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
-inline hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  ++g_pinned;
+  return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
+}
+inline hipError_t hipHostFree(void* p) {
+  --g_pinned;
+  std::free(p);
+  return hipSuccess;
+}
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = static_cast<int*>(std::malloc(4)); return hipSuccess; }

@@ -6,7 +6,7 @@
 #include <new>
 #include <vector>
 
-int g_fail_copies = 0;
+int g_fail_copies = 0, g_pinned = 0;
 static thread_local bool t_no_memory = false;   // operator new throws in this thread
 
 void* operator new(size_t n) {
@@ -36,6 +36,17 @@ int main() {
   pcx_internal::xfer_acquire();
   int bad = 0;
   const size_t M = (size_t)1 << 20;
+  // engines that come and go with a large result each allocate nothing pinned
+  for (int i = 0; i < 5; ++i) {
+    bad += check(24 * M, 7 * M, false, "one read an engine");
+    bad += g_pinned != 0;
+    pcx_internal::xfer_release();
+    pcx_internal::xfer_acquire();
+  }
+  bad += check(24 * M, 8 * M, false, "before the slots");
+  bad += g_pinned != 0;
+  bad += check(2 * M, 0, false, "the first through the slots");
+  bad += g_pinned != 1;
   for (size_t n : {(size_t)0, (size_t)1, M - 1, M, M + 1, 2 * M - 4095, 4 * M, 4 * M + 1, 5 * M + 77, 9 * M + 4097})
     for (size_t n2 : {(size_t)0, (size_t)3, M, 3 * M + 5}) {
       bad += check(n, n2, false, "threads");
@@ -46,7 +57,9 @@ int main() {
   bad += pcx_internal::copy_to_host(d.data(), 3 * M, nullptr, 0, s.data(), 0, nullptr) == hipSuccess;
   g_fail_copies = 0;
   bad += check(3 * M, 0, false, "after a failure");
+  bad += g_pinned != 1;
   pcx_internal::xfer_release();
+  bad += g_pinned != 0;
   std::printf(bad ? "failed\n" : "ok\n");
   return bad != 0;
 }

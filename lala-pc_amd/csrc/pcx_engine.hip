@@ -454,10 +454,25 @@ bool drains_branching(const pcx_batch* b, int32_t mode) {
   return mode == PCX_MODE_BATCHED && b->seeded && b->d_dirty && b->e->cfg.max_sweeps <= 0 && events_possible(b, mode);
 }
 
-// The lists of a drain: trails, then seeds.
-pcx_status ensure_trail(pcx_batch* b) {
-  if (!b->d_trail) PCX_HIP(hipMalloc(&b->d_trail, b->n_inst * (kTrailCap + kSeedCap) * sizeof(int32_t)));
-  if (!b->d_trail_n) PCX_HIP(hipMalloc(&b->d_trail_n, 2 * b->n_inst * sizeof(int32_t)));
+// The lists of a drain in one allocation (a search that makes its batches as it goes
+// has it on every first step): trails, seeds and their counts.  With the undo log of a
+// branching's drain, which takes no seeds, the seeds lie in the log's room: a run that
+// lists seeds starts from a loaded image, which ends what the log was kept for.
+pcx_status ensure_trail(pcx_batch* b, bool undo = false) {
+  static_assert(kSeedCap * sizeof(int32_t) <= kTrailCap * sizeof(int2), "the seeds fit the log");
+  const int64_t log = b->n_inst * kTrailCap * sizeof(int2), trail = b->n_inst * kTrailCap * sizeof(int32_t);
+  if (!b->d_trail) {
+    const int64_t before = undo ? log : b->n_inst * kSeedCap * (int64_t)sizeof(int32_t);
+    PCX_HIP(hipMalloc(&b->d_lists, before + trail + 2 * b->n_inst * sizeof(int32_t)));
+    if (undo) b->d_undo = reinterpret_cast<int2*>(b->d_lists);
+    b->d_seeds = reinterpret_cast<int32_t*>(b->d_lists);
+    b->d_trail = reinterpret_cast<int32_t*>(b->d_lists + before);
+    b->d_trail_n = reinterpret_cast<int32_t*>(b->d_lists + before + trail);
+  }
+  if (undo && !b->d_undo) {
+    PCX_HIP(hipMalloc(&b->d_log, log));
+    b->d_undo = b->d_log;
+  }
   return PCX_OK;
 }
 
@@ -998,7 +1013,7 @@ pcx_status run_batched(pcx_batch* b, const SeedPlan& plan, pcx_result* results, 
     const pcx_status ls = ensure_trail(b);
     if (ls != PCX_OK) return ls;
     if (base_seeded) {                   // a branching's seeds are bits in the rows
-      seeds = InstLists{b->d_trail + b->n_inst * kTrailCap, b->d_trail_n + b->n_inst, kSeedCap};
+      seeds = InstLists{b->d_seeds, b->d_trail_n + b->n_inst, kSeedCap};
       if (!counts) PCX_HIP(hipMemsetAsync(seeds.n, 0, b->n_inst * sizeof(int32_t), e->stream));
     }
   }
@@ -1482,9 +1497,8 @@ void pcx_batch_destroy(pcx_batch* b) {
   if (b->queue_graph) (void)hipGraphExecDestroy(b->queue_graph);
   if (b->plain_queue_graph) (void)hipGraphExecDestroy(b->plain_queue_graph);
   dfree(b->d_q); dfree(b->d_qctl);
-  dfree(b->d_diff); dfree(b->d_diff_val); dfree(b->d_unsat); dfree(b->d_trail); dfree(b->d_trail_n); dfree(b->d_bvar); dfree(b->d_seedctl); dfree(b->d_base); dfree(b->d_base_alt);
+  dfree(b->d_diff); dfree(b->d_diff_val); dfree(b->d_unsat); dfree(b->d_lists); dfree(b->d_log); dfree(b->d_bvar); dfree(b->d_seedctl); dfree(b->d_base); dfree(b->d_base_alt);
   dfree(b->d_ask);
-  dfree(b->d_undo);
   for (hipEvent_t ev : b->load_ev)
     if (ev) (void)hipEventDestroy(ev);
   delete b;
@@ -1817,23 +1831,24 @@ pcx_status pcx_batch_branch(pcx_batch* parent, pcx_batch* child, int32_t* var, i
   // more.  Without room for the log the image is written here.
   bool lazy = seeds && e->cfg.max_sweeps <= 0;
   if (lazy && !child->d_undo) {
-    lazy = ensure_trail(child) == PCX_OK &&
-           hipMalloc(&child->d_undo, child->n_inst * kTrailCap * sizeof(int2)) == hipSuccess;
+    lazy = ensure_trail(child, true) == PCX_OK;
     if (!lazy) (void)hipGetLastError();
-  }
-  if (seeds) {
-    pcx_status st = sync_table(e);
-    if (st == PCX_OK) st = ensure_event_buffers(child);
-    if (st == PCX_OK && !child->marks_clean) st = clear_marks(child);
-    if (st != PCX_OK) return st;
   }
   hipError_t he = launch_branch(parent->d_store, parent->nvars, parent->n_inst, d_var, child->d_store,
                                 lazy ? nullptr : child->d_image, child->d_image_empty, dom_of(e), e->stream);
   child->seeded = false;
+  // Behind the branch kernel, which hides what a first step allocates.  Without room
+  // for the marks the children are there all the same, unseeded.
+  pcx_status marked = PCX_OK;
   if (he == hipSuccess && seeds) {
-    he = launch_branch_seed(event_set(child), d_var, child->n_inst, e->stream);
-    child->marks_clean = false;
-    child->seeded = he == hipSuccess;
+    marked = sync_table(e);
+    if (marked == PCX_OK) marked = ensure_event_buffers(child);
+    if (marked == PCX_OK && !child->marks_clean) marked = clear_marks(child);
+    if (marked == PCX_OK) {
+      he = launch_branch_seed(event_set(child), d_var, child->n_inst, e->stream);
+      child->marks_clean = false;
+      child->seeded = he == hipSuccess;
+    }
   }
   if (he == hipSuccess && var)
     he = hipMemcpyAsync(var, d_var, parent->n_inst * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream);
@@ -1843,7 +1858,7 @@ pcx_status pcx_batch_branch(pcx_batch* parent, pcx_batch* child, int32_t* var, i
   pcx_status st = image_loaded(child, true);        // the branch wrote the children's emptiness
   child->seeded = seeded;
   child->image_absent = lazy && st == PCX_OK;
-  return st;
+  return marked != PCX_OK ? marked : st;
 }
 
 namespace {

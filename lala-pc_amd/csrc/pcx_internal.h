@@ -91,11 +91,13 @@ struct pcx_batch {
   hipEvent_t load_ev[2] = {nullptr, nullptr};
   int64_t diff_cap = 0;
   int32_t* d_unsat = nullptr;         // [table_n]
-  int32_t* d_trail = nullptr;         // [n_inst * kTrailCap] variables a drained run tightened,
-                                      // then [n_inst * kSeedCap] the drain's seeds
+  uint8_t* d_lists = nullptr;         // the allocation of the next three, and of the log if it came with them
+  int32_t* d_trail = nullptr;         // [n_inst * kTrailCap] variables a drained run tightened
+  int32_t* d_seeds = nullptr;         // [n_inst * kSeedCap] the drain's seeds (in the log's room)
   int32_t* d_trail_n = nullptr;       // [2 * n_inst]: the two lists' counts
   bool trail_valid = false;           // the stores are the image but for the trail's variables
   int2* d_undo = nullptr;             // [n_inst * kTrailCap] the values of the trail's variables before
+  int2* d_log = nullptr;              // its own allocation, where it came later
   bool image_absent = false;          // nothing holds the image but the stores themselves, or (after
                                       // a drained run) the stores and the undo log: a branching that
                                       // seeded a drain

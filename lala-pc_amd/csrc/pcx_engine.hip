@@ -1863,9 +1863,8 @@ pcx_status pcx_batch_branch(pcx_batch* parent, pcx_batch* child, int32_t* var, i
 
 namespace {
 // A formula tree list is well formed: known kinds, variables inside the
-// store, ternary opcodes, a stack within kTreeMaxDepth that ends each formula
+// store, ternary opcodes, a stack within kTreeDepth that ends each formula
 // with one value.
-constexpr int kTreeMaxDepth = 32;
 bool trees_valid(const int32_t* nodes, int64_t n_nodes, const int64_t* off, int64_t n_formulas,
                  int64_t nvars, std::string* why) {
   if (off[0] != 0 || off[n_formulas] != n_nodes) { *why = "offsets do not cover the nodes"; return false; }
@@ -1901,7 +1900,7 @@ bool trees_valid(const int32_t* nodes, int64_t n_nodes, const int64_t* off, int6
       }
       if (depth < pop) { *why = "node without its operands"; return false; }
       depth += push - pop;
-      if (depth > kTreeMaxDepth) { *why = "tree deeper than 32"; return false; }
+      if (depth > kTreeDepth) { *why = "tree deeper than 32"; return false; }
     }
     if (depth != 1) { *why = "formula leaves " + std::to_string(depth) + " values"; return false; }
   }

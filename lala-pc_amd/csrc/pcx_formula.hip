@@ -14,7 +14,7 @@
 //    one coalesced load, and the stack lies in LDS.  What bounds it: the copy's
 //    bytes from L2 and the latency of a node.
 //  - k_formula_ask: a thread per (store, formula), for few stores (their lanes
-//    would be idle).  Every variable is a gather and every lane follows its own
+//    would be idle) and few formulas (the copy would take longer).  Every variable is a gather and every lane follows its own
 //    nodes, the stack in scratch memory.
 // 50,000 formulas on 512 stores of 12,500 variables, half of them solutions:
 // 0.78 ms a thread per pair, 0.18 ms in lanes (and 0.02 for the copy).  On 16, 64
@@ -172,7 +172,7 @@ __device__ __forceinline__ int2 interpret(const int4* __restrict__ nodes, int64_
         ++j;                                       // the PROP_Z node
         break;
       }
-      default: break;                              // (validated on the host)
+      default: break;                              // (k_trees_check let none through)
     }
   }
   return s.top;
@@ -180,7 +180,6 @@ __device__ __forceinline__ int2 interpret(const int4* __restrict__ nodes, int64_
 
 namespace {
 
-constexpr int kTreeDepth = 32;         // the host refuses deeper trees
 constexpr int kGroup = kWave;          // stores per group of the interleaved copy
 constexpr int kPerWave = 8;            // formulas a wave asks per turn
 

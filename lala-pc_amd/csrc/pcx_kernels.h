@@ -422,11 +422,13 @@ hipError_t launch_ask(const Table& t, const int2* store, uint8_t* ent, int32_t* 
 hipError_t launch_formula_ask(const int4* nodes, const int64_t* off, int64_t n_formulas, const int2* store,
                               int64_t nvars, int64_t n_inst, int32_t* ok, hipStream_t st);
 // Whether a node list is well formed, formula by formula: verdict[0] (zeroed by
-// the caller) becomes 1 where one is not, verdict[1] the deepest stack.
+// the caller) becomes 1 where one is not, verdict[1] the deepest stack (at most
+// kTreeDepth in a well-formed one).
+constexpr int kTreeDepth = 32;
 hipError_t launch_trees_check(const int4* nodes, int64_t n_nodes, const int64_t* off, int64_t n_formulas,
                               int64_t nvars, int32_t* verdict, hipStream_t st);
 // The same over the stores' interleaved copy in groups of 64 (launch_interleave);
-// depth: the deepest stack of the trees, at most 32.
+// depth: the deepest stack of the trees, at most kTreeDepth.
 hipError_t launch_formula_lanes(const int4* nodes, const int64_t* off, int64_t n_formulas, int depth,
                                 const int2* shadow, int64_t nvars, int64_t n_inst, int32_t* ok, int cus,
                                 hipStream_t st);

@@ -41,8 +41,8 @@
 // A launch gives an instance kLocalLinks rounds and chase steps.  One that is not
 // at its fixpoint then stays unsettled (settled_at < 0), its store as far as it
 // came, and the host launches again: the instance goes on with every propagator
-// marked, and its counts with it.  So a launch ends (in about 10 ms an instance)
-// however slowly a store converges.
+// marked, and its counts with it.  So a launch ends (4,096 steps of a chase take 6
+// ms) however slowly a store converges.
 //
 // What bounds it: the depth of the propagation times the latency of one link
 // (operands and meets in LDS, the adjacency from L2, and the instructions of one
@@ -64,14 +64,14 @@ constexpr int kWalkVars = kWave / kWalkLanes;
 constexpr int kChasePerWave = 8;         // marks a wave chases at most when a chase starts
 constexpr int kLocalLinks = 4096;      // rounds and chase steps of an instance in one launch
 constexpr int64_t kLocalStatic = 256;  // static LDS of the kernel (counters), at most
-constexpr int kHubRounds = 2;
-// A walk of 16 lanes takes about 0.025 us an entry, a sweep by the workgroup 1.3 us
-// and 0.001 a propagator.
+constexpr int kHubRounds = 2;          // dense rounds after hubs before the instance is left
+// Propagators of a variable from which on it is a hub: a walk of 16 lanes takes about
+// 0.025 us an entry, a sweep by the workgroup 1.3 us and 0.001 a propagator.
 int32_t hub_degree(int64_t n_props) { return (int32_t)(96 + std::min<int64_t>(n_props / 32, 1024)); }
 constexpr int32_t kResumeMax = 1 << 30;  // rounds a resumed run is taken to have had, at most (they are counted in 32 bits)
 
 // Workgroups of 1,024 threads (batches that leave compute units idle: the
-// dense rounds are then as wide as one unit allows) or 256 (larger batches:
+// dense rounds are then as wide as one unit allows) or 512 (larger batches:
 // other instances fill the unit).
 constexpr int kWide = 1024, kNarrow = 512;
 

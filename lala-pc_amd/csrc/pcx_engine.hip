@@ -123,7 +123,8 @@ pcx_status ensure_adjacency(pcx_engine* e) {
     PCX_HIP(he);
     PCX_HIP(se);
   } else {
-    PCX_HIP(hipMemset(e->d_adj_off, 0, (V + 1) * sizeof(int32_t)));
+    PCX_HIP(hipMemsetAsync(e->d_adj_off, 0, (V + 1) * sizeof(int32_t), e->stream));
+    PCX_HIP(hipStreamSynchronize(e->stream));
   }
   e->adj_vars = V;
   e->adj_n = total;

@@ -191,6 +191,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
     }
 
     int32_t failed_at = start_failed ? -1 : kNoFail, r = r0;
+    const int32_t r_end = r0 + kLocalLinks;
     bool unsettled = false;
     int hubs = 0;                                    // rounds and chases that tightened one
     int nt0 = 0, nt = 0;                             // (a launch's share fits: kLocalLinks bounds it)
@@ -240,7 +241,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       }
     };
     while (!start_failed) {
-      unsettled = r - r0 >= kLocalLinks;
+      unsettled = r >= r_end;
       if (unsettled) break;
       // ---- round r: (B)
       const int cur = r & 1, nx = cur ^ 1;
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
           z = t.z[q];
         }
       }
-      for (const int left = kLocalLinks - (r - r0); steps < left && __ballot(q >= 0); ++steps) {
+      for (; steps < r_end - r && __ballot(q >= 0); ++steps) {
         const int32_t stop = __hip_atomic_load(&s_fail, __ATOMIC_RELAXED, WG);   // arrives with the operands
         tx = ty = tz = false;
         if (q >= 0) {

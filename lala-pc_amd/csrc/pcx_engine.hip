@@ -548,6 +548,12 @@ struct SeedPlan {
   bool seeded = false;
   int64_t n_diff = 0, n_unsat = 0;
 };
+bool few_seeds(const pcx_batch* b) {          // by the probe of the image
+  if (b->probe_diff < 0) return false;
+  const int64_t per_var = 3 * b->table_n / std::max<int64_t>(b->nvars, 1) + 1;   // mean adjacency
+  const int64_t pairs = b->h_off.empty() ? b->n_inst * b->table_n : b->h_off.back();
+  return (b->probe_diff * per_var + b->probe_unsat * b->n_inst) * 16 <= pairs;
+}
 pcx_status plan_seed(pcx_batch* b, SeedPlan* plan) {
   *plan = SeedPlan{};
   pcx_engine* e = b->e;
@@ -572,12 +578,7 @@ pcx_status plan_seed(pcx_batch* b, SeedPlan* plan) {
     b->probe_version = e->version;
     b->probe_valid = true;
   }
-  if (b->probe_diff < 0) return PCX_OK;
-  const int64_t n_diff = b->probe_diff, n_unsat = b->probe_unsat;
-  const int64_t per_var = 3 * b->table_n / std::max<int64_t>(b->nvars, 1) + 1;   // mean adjacency
-  const int64_t pairs = b->h_off.empty() ? b->n_inst * b->table_n : b->h_off.back();
-  if ((n_diff * per_var + n_unsat * b->n_inst) * 16 > pairs) return PCX_OK;
-  *plan = SeedPlan{true, n_diff, n_unsat};
+  if (few_seeds(b)) *plan = SeedPlan{true, b->probe_diff, b->probe_unsat};
   return PCX_OK;
 }
 
@@ -600,6 +601,13 @@ pcx_status plan_seed(pcx_batch* b, SeedPlan* plan) {
 // 0.22, 0.46, 1.06, 4.88 / 0.43, 0.76, 1.42, 6.23 there; 1,000 of 4,000 variables, 6
 // and 25% of 100,003: 1.95 and 1.77 here, 0.21 and 0.91 there).
 constexpr int64_t kLocalBatchProps = (int64_t)1 << 17;
+// Bitset batches in persistent mode: small stores settle in a dozen full sweeps of
+// little more than a step per thread, which marks and lists only slow down, unless the
+// stores start near their fixpoints (1,000 stores with 2,000, 4,000, 6,000, 12,000 and
+// 16,000 propagators, unpropagated: 1.04, 0.84, 1.40, 2.02, 1.85 ms here, 0.47, 0.69,
+// 1.30, 1.96, 2.16 in full sweeps; splits of the root fixpoint: 0.12, 0.12, 0.16, 0.21,
+// 0.25 here, 0.14, 0.16, 0.29, 0.41, 0.51 there).
+constexpr int64_t kLocalBitsProps = 12 * 1024;
 bool local_wanted(const pcx_batch* b, int32_t mode, bool seeded) {
   const pcx_config& c = b->e->cfg;
   if (b->no_local) return false;
@@ -608,7 +616,11 @@ bool local_wanted(const pcx_batch* b, int32_t mode, bool seeded) {
   if (c.lds_mode == 0 || c.max_sweeps > 0 || c.event_driven == 0 || 3 * b->table_n >= ((int64_t)1 << 31) ||
       !local_fits(c.device, b->nvars, b->table_n))
     return false;
-  if (mode == PCX_MODE_PERSISTENT) return b->h_off.empty() || 3 * b->h_off.back() >= b->n_inst * b->table_n;
+  if (mode == PCX_MODE_PERSISTENT) {
+    if (!b->h_off.empty() && 3 * b->h_off.back() < b->n_inst * b->table_n) return false;
+    return c.domain == PCX_DOMAIN_INTERVAL || b->table_n >= kLocalBitsProps ||
+           (b->run_from_image && b->probe_valid && b->probe_version == b->e->version && few_seeds(b));
+  }
   return mode == PCX_MODE_BATCHED && c.domain == PCX_DOMAIN_INTERVAL && c.event_driven < 0 &&
          c.props_per_wave == 0 && c.lockstep < 0 && c.mark_queue < 0 && !seeded && !b->seeded &&
          b->table_n <= kLocalBatchProps;

@@ -28,7 +28,16 @@
 // pays once most propagators are settled: a few plain sweeps come first (one
 // fixpoint of 200,000 / 4,000,000 propagators with 1, 2, 4, 8 and 16 of them:
 // 0.84 / 3.45, 0.83 / 3.20, 0.77 / 3.06, 0.76 / 3.46 and 0.79 / 4.19 ms; plain and
-// marked sweeps alone 1.92 / 6.27).  Early chases cut after 1 to 8 links instead
+// marked sweeps alone 1.92 / 6.27).  Stores that settle in a few more sweeps need no
+// chase, which takes longer the more it finds to do: eight sweeps up to a million
+// propagators (chains of 6, 10, 20 and 200 in 1,000,000 with 4 / 8 / plain sweeps
+// alone: 750 / 513 / 617, 850 / 600 / 647, 920 / 925 / 735 and 1,260 / 1,330 / 2,890
+// us; in 500,000: 493 / 333 / 375, 540 / 452 / 391, 575 / 545 / 517 and 920 / 930 /
+// 2,080), four beyond, where a plain sweep costs more (1,400,000, the same chains
+// but the first: 1,098 / 800 / 1,411, then 1,210 / 1,280 / 2,202 with chains of 30,
+// 1,533 / 1,700 / 5,092).  Between 350,000 and a million propagators, stores of 10 to
+// 30 sweeps still take longer than by plain sweeps, by a third at most: a wave ends
+// one chase before it takes its next 64, and each wave has several.  Early chases cut after 1 to 8 links instead
 // of the plain sweeps took 1.1-1.4 / 4.4-7.7 ms; 2, 3 or 7 workgroups per compute
 // unit and 16 lanes per variable measured the same, 4 lanes 0.87 / 3.2.
 #include "pcx_device.h"

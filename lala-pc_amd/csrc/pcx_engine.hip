@@ -886,10 +886,11 @@ pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats, int32_
         if (q[kQStop] == 2) { s = q[kQAt]; break; }      // bitmap sweeps from sweep s on
       }
     }
+    const int after = pcx_internal::chase_after(b->table_n);
     for (; !done;) {
       // Full sweeps are timed one by one; consecutive marked sweeps as one span.
       int n_marked = 0;
-      const int count = b->chase ? pcx_internal::chase_count(s, group) : group;
+      const int count = b->chase ? pcx_internal::chase_count(s, after, group) : group;
       for (int g = 0; g < count; ++g, ++s) {
         if (e->cfg.max_sweeps > 0 && s >= e->cfg.max_sweeps) break;
         const bool marked = b->events && (s > 0 || b->seeded_run);
@@ -901,7 +902,7 @@ pcx_status run_plain(pcx_batch* b, pcx_result* results, pcx_stats* stats, int32_
                                             e->stream));
           ++n_marked;
         } else {
-          if (b->chase && s >= pcx_internal::kChaseAfter)
+          if (b->chase && s >= after)
             PCX_HIP(launch_sweep_chase(tk, st, s, f, b->d_tight, e->d_adj_off, e->d_adj_rec, dom_of(e),
                                        pcx_internal::device_cus(e->cfg.device), e->stream));
           else

@@ -158,13 +158,14 @@ bool single_local(const pcx_engine* e, int64_t nvars);
 hipError_t launch_single(const pcx_engine* e, int32_t* lb, int32_t* ub, int64_t nvars, pcx::InstFlags* flags,
                          bool resume);
 bool chase_wanted(const pcx_engine* e);       // plain runs of one store chase
-constexpr int kChaseAfter = 4;                // plain sweeps before the first chase (see pcx_chase.hip)
+// plain sweeps before the first chase of a table (see pcx_chase.hip)
+inline int chase_after(int64_t n_props) { return n_props <= (1 << 20) ? 8 : 4; }
 // Sweeps queued at sweep s of a run that chases before the host looks: mostly the
 // first chase finds the fixpoint and the second is quiet; a run that takes more
 // (variables too widely named to be chased) is looked at as rarely as other runs.
-inline int chase_count(int32_t s, int group) {
-  if (s == 0) return kChaseAfter + 2;
-  return s < kChaseAfter + 8 ? 2 : group;
+inline int chase_count(int32_t s, int after, int group) {
+  if (s == 0) return after + 2;
+  return s < after + 8 ? 2 : group;
 }
 pcx_result single_result(const pcx_engine* e, const pcx::InstFlags& f);
 }  // namespace pcx_internal

@@ -124,7 +124,7 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   PCX_HIP(launch_store_check_empty(d_store, nvars, 1, d_flags, dom, s));
 
   // Full sweeps, the flags read back every `group` sweeps (as the plain mode
-  // does), until a sweep changed nothing or the store failed; from the fifth on
+  // does), until a sweep changed nothing or the store failed; after the first few
   // they chase what they tighten when an earlier pcx_fixpoint left the adjacency
   // records.
   const bool chase = e->d_adj_rec && e->adj_rec_version == e->version && pcx_internal::chase_wanted(e);
@@ -140,11 +140,12 @@ pcx_status pcx_fixpoint_noalloc(pcx_engine* e, int32_t* d_lb, int32_t* d_ub, int
   const int64_t maxs = e->cfg.max_sweeps;
   InstFlags hf{};
   int32_t sw = 0;
+  const int after = pcx_internal::chase_after(m);
   for (;;) {
-    const int count = chase ? pcx_internal::chase_count(sw, group) : group;
+    const int count = chase ? pcx_internal::chase_count(sw, after, group) : group;
     for (int g = 0; g < count; ++g, ++sw) {
       if (maxs > 0 && sw >= maxs) break;
-      if (chase && sw >= pcx_internal::kChaseAfter)
+      if (chase && sw >= after)
         PCX_HIP(launch_sweep_chase(t, d_store, sw, d_flags, d_tight, e->d_adj_off, e->d_adj_rec, dom,
                                    pcx_internal::device_cus(e->cfg.device), s));
       else

@@ -739,6 +739,7 @@ pcx_status run_local(pcx_batch* b, int32_t mode, pcx_result* results, pcx_stats*
   job.adj = e->d_adj_rec;
   job.member = b->h_off.empty() ? nullptr : b->d_member;
   job.words = bitmap_words(b);
+  job.sweeps = mode != PCX_MODE_PLAIN && e->cfg.domain == PCX_DOMAIN_INTERVAL;
   std::vector<InstFlags> flags;
   const double load_ms = b->load_ms;        // (collect hands it out once)
   for (;;) {

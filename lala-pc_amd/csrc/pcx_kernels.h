@@ -349,6 +349,7 @@ struct LocalJob {
   const uint32_t* member;   // [n_inst * words], or nullptr: every propagator
   int64_t words;
   bool resume;              // go on from the stores and flags of the last launch
+  bool sweeps;              // whoever launches goes on with k_persistent where that serves an instance better
   int32_t hub;              // (set by launch_local) variables of a larger degree are not walked
 };
 constexpr int32_t kLocalLeft = -2;

@@ -12,7 +12,8 @@
 // of lanes walk the adjacency of the listed variables and mark the instance's
 // propagators, each new mark also listed for the next round.  A list that
 // overflows makes the next round dense; variables that overflow theirs, or that are
-// more than a sixteenth of the propagators, mark every propagator.
+// more than a sixteenth of the propagators, mark every propagator; an instance of a
+// batch of intervals that has kManyRounds such rounds in a row is left to sweeps, too.
 //
 // Chase, once few marks are left: each wave propagates its share of them
 // without barriers.  A lane holds one propagator's record (position, operands)
@@ -71,6 +72,13 @@ constexpr int64_t kLocalStatic = 256;  // static LDS of the kernel (counters), a
 // full sweeps 193, 276, 2,771); 1,000 with 16,000 propagators, 200 deep, 990, 974
 // (986; 1,065; 5,931).
 constexpr int kManyShift = 4, kManyLeast = 64;
+// Such rounds in a row before an instance is left to sweeps, whose rounds are shorter
+// and which more workgroups run at a time (256 / 1,000 stores in which chains of 100
+// rise by one a round, 4,000 and 16,000 propagators: 0.77 / 2.36 and 2.40 / 14.8 ms
+// here, 0.65 / 1.35 and 2.17 / 8.7 left after 4, 0.66 / 1.47 and 2.25 / 9.2 after 8,
+// 0.71 / 1.67 and 2.39 / 10.1 after 16, 0.60 / 1.16 and 2.05 / 8.0 in sweeps alone;
+// generated networks, 1 to 200 deep: the same).
+constexpr int kManyRounds = 4;
 constexpr int kHubRounds = 2;          // dense rounds after hubs before the instance is left
 // Propagators of a variable from which on it is a hub: a walk of 16 lanes takes about
 // 0.025 us an entry, a sweep by the workgroup 1.3 us and 0.001 a propagator.
@@ -201,6 +209,8 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
     const int32_t r_end = r0 + kLocalLinks;
     bool unsettled = false;
     int hubs = 0;                                    // rounds and chases that tightened one
+    int many = 0;                                    // rounds in a row that marked everything
+    bool left = false;
     int nt0 = 0, nt = 0;                             // (a launch's share fits: kLocalLinks bounds it)
     int ne = 0;                                      // evaluations after round 0
     // Evaluate one propagator on the LDS store; which operands it tightened.
@@ -313,7 +323,9 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
         for (int32_t w = tid; w < W; w += B) bm[w] = member_word(w);
         for (int32_t w = tid; w < VW; w += B) vbm[w] = 0;
         if (tid == 0) s_over[nx] = 1;
+        left = job.sweeps && ++many > kManyRounds;
       } else {
+        many = 0;
         // sixteen lanes per variable when that takes one pass, else eight
         const int lg = ntv * 16 <= B ? 4 : 3;
         const int sub = tid & ((1 << lg) - 1);
@@ -332,10 +344,11 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
         }
       }
       ++r;
+      if (left) break;
       __syncthreads();                               // every mark is set and listed
       if (s_hub) {
-        unsettled = ++hubs > kHubRounds;
-        if (unsettled) break;
+        left = ++hubs > kHubRounds;
+        if (left) break;
         __syncthreads();                             // every wave has read it
         mark_everything();
         __syncthreads();
@@ -440,8 +453,9 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       if (s_fail) { failed_at = r; break; }
       const bool hub = s_chub != 0;
       hubs += hub;
-      unsettled = s_out != 0 || hubs > kHubRounds;
-      if (unsettled || !(hub || s_over[cur])) break; // no marks left anywhere: the fixpoint
+      left = hubs > kHubRounds;
+      unsettled = s_out != 0;
+      if (left || unsettled || !(hub || s_over[cur])) break; // no marks left anywhere: the fixpoint
       // Marks that found a stack full: a dense round (of the parity r has now).
       __syncthreads();                               // every wave has read the flags
       if (hub) {
@@ -481,7 +495,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
         f->failed_at = failed_at;
         f->done_at = r;
         f->marked_evals += (int64_t)s_sum[2];
-        f->settled_at = !unsettled ? r : hubs > kHubRounds ? kLocalLeft : -1;
+        f->settled_at = left ? kLocalLeft : unsettled ? -1 : r;
       }
       if (job.tight) {
         const int at = slot & (kTightSlots - 1);

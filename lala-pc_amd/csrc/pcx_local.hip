@@ -75,9 +75,10 @@ constexpr int kManyShift = 4, kManyLeast = 64;
 // Such rounds in a row before an instance is left to sweeps, whose rounds are shorter
 // and which more workgroups run at a time (256 / 1,000 stores in which chains of 100
 // rise by one a round, 4,000 and 16,000 propagators: 0.77 / 2.36 and 2.40 / 14.8 ms
-// here, 0.65 / 1.35 and 2.17 / 8.7 left after 4, 0.66 / 1.47 and 2.25 / 9.2 after 8,
+// here, 0.64 / 1.31 and 2.13 / 8.6 left after 4, 0.66 / 1.47 and 2.25 / 9.2 after 8,
 // 0.71 / 1.67 and 2.39 / 10.1 after 16, 0.60 / 1.16 and 2.05 / 8.0 in sweeps alone;
-// generated networks, 1 to 200 deep: the same).
+// generated networks, 1 to 200 deep: the same).  Counted in LDS: in registers every
+// wave's count cost a spill and 2 to 5% of the chases.
 constexpr int kManyRounds = 4;
 constexpr int kHubRounds = 2;          // dense rounds after hubs before the instance is left
 // Propagators of a variable from which on it is a hub: a walk of 16 lanes takes about
@@ -146,8 +147,10 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
   __shared__ int32_t s_empty;                        // empty as loaded: no round writes it, a late wave may still read it
   __shared__ int32_t s_ntv[2], s_n[2], s_over[2];    // by parity of the round
   __shared__ int32_t s_out;                          // a wave ran out of steps
+  __shared__ int32_t s_many;                         // rounds in a row that marked everything (the first thread's)
   __shared__ int32_t s_hub, s_chub;                  // a hub was tightened in a round, in a chase (a
-                                                     // late wave reads the one while the other is set)
+                                                     // late wave reads the one while the other is set);
+                                                     // s_hub also ends an instance that is left
   __shared__ unsigned long long s_sum[3];
   const int tid = threadIdx.x, lane = lane_id(), wave = uni(tid / kWave);
   const int32_t V = (int32_t)job.nvars, P = (int32_t)t.n;
@@ -184,7 +187,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       if (mrow) return mrow[w];
       return (w == W - 1 && (P & 31)) ? (1u << (P & 31)) - 1u : ~0u;
     };
-    if (tid == 0) { s_fail = 0; s_empty = 0; s_chg = 0; s_steps = 0; s_ntv[0] = s_ntv[1] = 0; s_n[0] = s_n[1] = 0; s_over[r0 & 1] = 1; s_over[(r0 & 1) ^ 1] = 0; s_out = s_hub = s_chub = 0; }
+    if (tid == 0) { s_fail = 0; s_empty = 0; s_chg = 0; s_steps = 0; s_ntv[0] = s_ntv[1] = 0; s_n[0] = s_n[1] = 0; s_over[r0 & 1] = 1; s_over[(r0 & 1) ^ 1] = 0; s_out = s_hub = s_chub = s_many = 0; }
     if (tid < 3) s_sum[tid] = 0;
     __syncthreads();                                 // s_slot is read; the counters are set
     if (!start_failed) {
@@ -209,8 +212,6 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
     const int32_t r_end = r0 + kLocalLinks;
     bool unsettled = false;
     int hubs = 0;                                    // rounds and chases that tightened one
-    int many = 0;                                    // rounds in a row that marked everything
-    bool left = false;
     int nt0 = 0, nt = 0;                             // (a launch's share fits: kLocalLinks bounds it)
     int ne = 0;                                      // evaluations after round 0
     // Evaluate one propagator on the LDS store; which operands it tightened.
@@ -322,10 +323,12 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       if (ntv > min(kLocalVars, max(P >> kManyShift, kManyLeast))) {   // many, or some were lost: mark everything
         for (int32_t w = tid; w < W; w += B) bm[w] = member_word(w);
         for (int32_t w = tid; w < VW; w += B) vbm[w] = 0;
-        if (tid == 0) s_over[nx] = 1;
-        left = job.sweeps && ++many > kManyRounds;
+        if (tid == 0) {
+          s_over[nx] = 1;
+          if (job.sweeps && ++s_many > kManyRounds) s_hub = kHubRounds + 1;
+        }
       } else {
-        many = 0;
+        if (tid == 0) s_many = 0;
         // sixteen lanes per variable when that takes one pass, else eight
         const int lg = ntv * 16 <= B ? 4 : 3;
         const int sub = tid & ((1 << lg) - 1);
@@ -344,11 +347,11 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
         }
       }
       ++r;
-      if (left) break;
       __syncthreads();                               // every mark is set and listed
       if (s_hub) {
-        left = ++hubs > kHubRounds;
-        if (left) break;
+        hubs += s_hub;
+        unsettled = hubs > kHubRounds;
+        if (unsettled) break;
         __syncthreads();                             // every wave has read it
         mark_everything();
         __syncthreads();
@@ -453,9 +456,8 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
       if (s_fail) { failed_at = r; break; }
       const bool hub = s_chub != 0;
       hubs += hub;
-      left = hubs > kHubRounds;
-      unsettled = s_out != 0;
-      if (left || unsettled || !(hub || s_over[cur])) break; // no marks left anywhere: the fixpoint
+      unsettled = s_out != 0 || hubs > kHubRounds;
+      if (unsettled || !(hub || s_over[cur])) break; // no marks left anywhere: the fixpoint
       // Marks that found a stack full: a dense round (of the parity r has now).
       __syncthreads();                               // every wave has read the flags
       if (hub) {
@@ -495,7 +497,7 @@ __global__ __launch_bounds__(B, (local_min_waves<D, B>())) void k_local(Table t,
         f->failed_at = failed_at;
         f->done_at = r;
         f->marked_evals += (int64_t)s_sum[2];
-        f->settled_at = left ? kLocalLeft : unsettled ? -1 : r;
+        f->settled_at = !unsettled ? r : hubs > kHubRounds ? kLocalLeft : -1;
       }
       if (job.tight) {
         const int at = slot & (kTightSlots - 1);
